@@ -672,9 +672,17 @@ int32_t lbmoe_dense_mlp(const void* gate_proj, const void* up_proj, const void* 
     void* actq = at<void>(workspace, w, R_ACTQ);
     float* acts = at<float>(workspace, w, R_ACTS);
     LBMOE_TRY(launch_quant_groups_fp8(x, T, H, H, xq, xs, s));
+    if (dense_tiled_fp8_supported(gw, T, Imax, xq, actq, out)) {
+      LBMOE_TRY(launch_dense_tiled_fp8(gw, xq, xs, T, Imax, actq, acts, out, s));
+      return LBMOE_OK;
+    }
     LBMOE_TRY(launch_gate_up_fp8(gw, xq, xs, nullptr, nullptr, nullptr, T, 1, Imax, act, s));
     LBMOE_TRY(launch_quant_groups_fp8(act, T, Imax, Imax, actq, acts, s));
     LBMOE_TRY(launch_down_fp8(gw, actq, acts, Imax, nullptr, nullptr, T, 1, out, s));
+    return LBMOE_OK;
+  }
+  if (dense_tiled_supported(gw, x, T, Imax, act, out)) {
+    LBMOE_TRY(launch_dense_tiled(gw, x, T, Imax, act, out, s));
     return LBMOE_OK;
   }
   LBMOE_TRY(launch_gate_up_bf16(gw, x, nullptr, nullptr, nullptr, T, 1, Imax, act, s));

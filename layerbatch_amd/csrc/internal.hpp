@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <initializer_list>
+
 #include "../../include/lbmoe.h"
 
 namespace lbmoe {
@@ -254,7 +256,34 @@ hipError_t launch_gate_up_tiled_fp8(const GroupWeights& gw, const void* xq, cons
 hipError_t launch_down_tiled_fp8(const GroupWeights& gw, const void* actq, const float* acts,
                                  int act_ld, const int32_t* tiles, int max_tiles, void* out,
                                  hipStream_t s);
+// The dense MLP on LDS-tiled GEMMs (weights gw.sh_*, act rows act_ld apart): batches of at least
+// kDenseTiledMinTokens tokens with 16-byte aligned operands within the buffer copies' range. Up to
+// 28 tokens the streaming kernels run two token tiles per pass (H = 2048, Is = 512: T=24 9.4 us
+// against 11.4), above four (T=32 12.4 against 11.5). A tile shape is taken where it gives at least
+// kDenseMinWorkgroups workgroups (launch_dense_gemm).
+constexpr int64_t kDenseTiledMinTokens = 29;
+constexpr int64_t kDenseMinWorkgroups = 160;
+bool dense_tiled_supported(const GroupWeights& gw, const void* x, int64_t T, int act_ld,
+                           const void* act, const void* out);
+hipError_t launch_dense_tiled(const GroupWeights& gw, const void* x, int64_t T, int act_ld,
+                              void* act, void* out, hipStream_t s);
+// fp8: xq, xs are x's codes and scales; gate_up writes the act's.
+bool dense_tiled_fp8_supported(const GroupWeights& gw, int64_t T, int act_ld, const void* xq,
+                               const void* actq, const void* out);
+hipError_t launch_dense_tiled_fp8(const GroupWeights& gw, const void* xq, const float* xs,
+                                  int64_t T, int act_ld, void* actq, float* acts, void* out,
+                                  hipStream_t s);
 bool tiled_router_supported(int E, int H);
+// whether launch_router_logits_tiled takes 64 x 64 tiles with the k range split
+bool router_small_tiles(const void* x, const void* wg, const void* logits, int64_t T, int E,
+                        int H);
+// Whether every pointer is 16-byte aligned, as the direct global -> LDS copies and whole-row
+// stores of the tiles that callers' tensors reach are kept.
+inline bool aligned16(std::initializer_list<const void*> ptrs) {
+  uintptr_t bits = 0;
+  for (const void* p : ptrs) bits |= reinterpret_cast<uintptr_t>(p);
+  return (bits & 15) == 0;
+}
 // whether launch_router_logits runs the LDS-tiled router for this batch
 bool router_is_tiled(int64_t T, int E, int H);
 // Router logits + selection + the permutation's count pass in one launch (E <= 128), then the

@@ -52,7 +52,8 @@ __device__ __forceinline__ i32x8 cat8(u32x4 lo, u32x4 hi) {
 // PERSIST: called from the persistent kernel's item loop, where the thread index goes through
 // an empty asm, so the per-lane arithmetic is redone per item rather than hoisted out of the loop
 // and held in registers across it.
-template <bool GATEUP, class S, bool PERSIST = false>
+// DENSE: the dense MLP, as in the bf16 kernels: no non-temporal weight copies or output stores.
+template <bool GATEUP, class S, bool PERSIST = false, bool DENSE = false>
 __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
                                                  const uint8_t* __restrict__ src,
                                                  const float* __restrict__ src_sc, int src_ld,
@@ -179,7 +180,7 @@ __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
     for (int t = 0; t < kN16; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // narrow and tiny tiles' weight copies are non-temporal, as in the bf16 kernel
-  constexpr int kWeightPolicy = S::kWT < kWM ? 2 : 0;
+  constexpr int kWeightPolicy = !DENSE && S::kWT < kWM ? 2 : 0;
   __amdgpu_buffer_rsrc_t ars[kALoads];
 #pragma unroll
   for (int i = 0; i < kALoads; ++i) ars[i] = raw_rsrc(abase[i]);
@@ -362,7 +363,7 @@ __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
       }
     }
   } else {
-    store_staged<kCols, kWT, true>(lds, static_cast<uint16_t*>(dst), dst_ld, row0, r0, n, c0);
+    store_staged<kCols, kWT, !DENSE>(lds, static_cast<uint16_t*>(dst), dst_ld, row0, r0, n, c0);
   }
 }
 
@@ -422,7 +423,70 @@ void tiled_fp8_persistent_kernel(GroupWeights gw, const uint8_t* __restrict__ sr
   }
 }
 
+// The dense SwiGLU MLP: (token tile, weight tile) items of one group, no tile list. The streaming
+// kernels reload the weights for every 64 tokens and leave the act's quantisation to a launch of its
+// own: H = 2048, Is = 512, T=777 32.0 -> 21 us, T=16384 387 -> 95 us, bit-exact.
+template <bool GATEUP, class S>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void dense_tiled_fp8_kernel(GroupWeights gw, const uint8_t* __restrict__ src,
+                            const float* __restrict__ src_sc, int src_ld, int T, int n_wtiles,
+                            void* __restrict__ dst, int dst_ld, float* __restrict__ dst_sc) {
+  __shared__ u32x4 lds[kRingU4];
+  __shared__ float scl[kActScales + kWScales];
+  const int item = xcd_item(blockIdx.x, (T + S::kWT - 1) / S::kWT * n_wtiles);
+  if (item < 0) return;
+  const int ti = item / n_wtiles, wt = item - ti * n_wtiles;
+  tile_product_fp8<GATEUP, S, false, true>(gw, src, src_sc, src_ld, nullptr, gw.E, ti * S::kWT, T,
+                                           0, wt, dst, dst_ld, dst_sc, lds, scl);
+}
+
+template <bool GATEUP, class S>
+static hipError_t launch_dense_shape(const GroupWeights& gw, const void* src, const float* src_sc,
+                                     int src_ld, int64_t T, void* dst, int dst_ld, float* dst_sc,
+                                     hipStream_t s) {
+  const int n_wtiles = GATEUP ? gw.Is / (kWM / 2) : gw.H / kWM;
+  const int64_t n_ttiles = (T + S::kWT - 1) / S::kWT;
+  dense_tiled_fp8_kernel<GATEUP, S><<<round8(n_ttiles * n_wtiles), kThreads, 0, s>>>(
+      gw, static_cast<const uint8_t*>(src), src_sc, src_ld, static_cast<int>(T), n_wtiles, dst,
+      dst_ld, dst_sc);
+  return hipGetLastError();
+}
+
+// Tile of one dense GEMM: the widest whose workgroups occupy most CUs, as for bf16. A 256-row
+// gate_up tile is one quantisation group of the act, so its epilogue can write the down GEMM's codes.
+// Measured (us, quantisation of x + gate_up of H = 2048, Is = 512): T=777 tiny / narrow / wide 16.7 /
+// 22.3 / 33.4, T=8192 40.7 / 34.4 / 42.1, T=16384 75.4 / 63.9 / 56.1; down likewise.
+template <bool GATEUP>
+static hipError_t launch_dense_gemm(const GroupWeights& gw, const void* src, const float* src_sc,
+                                    int src_ld, int64_t T, void* dst, int dst_ld, float* dst_sc,
+                                    hipStream_t s) {
+  const int n_wtiles = GATEUP ? gw.Is / (kWM / 2) : gw.H / kWM;
+  auto enough = [&](int t) { return (T + t - 1) / t * n_wtiles >= kDenseMinWorkgroups; };
+  if (enough(Wide::kWT))
+    return launch_dense_shape<GATEUP, Wide>(gw, src, src_sc, src_ld, T, dst, dst_ld, dst_sc, s);
+  if (enough(Narrow::kWT))
+    return launch_dense_shape<GATEUP, Narrow>(gw, src, src_sc, src_ld, T, dst, dst_ld, dst_sc, s);
+  return launch_dense_shape<GATEUP, Tiny>(gw, src, src_sc, src_ld, T, dst, dst_ld, dst_sc, s);
+}
+
 }  // namespace f8t
+
+bool dense_tiled_fp8_supported(const GroupWeights& gw, int64_t T, int act_ld, const void* xq,
+                               const void* actq, const void* out) {
+  return T >= kDenseTiledMinTokens && gw.H % kWM == 0 && gw.Is % (kWM / 2) == 0 &&
+         gw.H / 128 <= f8t::kMaxKBlocks && gw.Is / 128 <= f8t::kMaxKBlocks &&
+         fp8_tiled_offsets_fit(T, T, gw.H, act_ld) &&
+         aligned16({xq, actq, out, gw.sh_gate, gw.sh_up, gw.sh_down});
+}
+
+hipError_t launch_dense_tiled_fp8(const GroupWeights& gw, const void* xq, const float* xs,
+                                  int64_t T, int act_ld, void* actq, float* acts, void* out,
+                                  hipStream_t s) {
+  const hipError_t e =
+      f8t::launch_dense_gemm<true>(gw, xq, xs, gw.H, T, actq, act_ld, acts, s);
+  if (e != hipSuccess) return e;
+  return f8t::launch_dense_gemm<false>(gw, actq, acts, act_ld, T, out, gw.H, nullptr, s);
+}
 
 bool tiled_fp8_supported(const GroupWeights& gw, int64_t T, int64_t rows) {
   // the copies address operands with byte offsets below 2^31 from a weight matrix, xq or actq

@@ -65,6 +65,13 @@ using RouterShape128 = TileShape<4, 1, 1, 64, 3>;
 // which moves fewer operand bytes per flop than 64-token tiles
 using RouterShapeTall = TileShape<2, 4, 1, 64, 3>;
 constexpr int64_t kRouterTallMinWorkgroups = 256;
+// dense MLP (dense_tiled_kernel), besides Wide and Narrow: 2 x 4 waves of 64 x 32 (128 x 128),
+// 2 x 2 waves of 64 x 32 (128 x 64, two workgroups per CU) and 1 x 2 waves of 64 x 32 (64 x 64) for
+// KS groups of waves
+using Dense128 = TileShape<2, 2, 1, 64, 3>;
+using Dense128x64 = TileShape<2, 2, 1, 64, 3, 3, 4>;
+using Dense64 = TileShape<1, 2, 1, 64, 3, 3, 2>;     // KS = 2: 96 KB
+using Dense64x4 = TileShape<1, 2, 1, 64, 2, 2, 2>;   // KS = 4: 128 KB
 constexpr int kLdsU4 = Wide::kRingU4 > Narrow::kRingU4 ? Wide::kRingU4 : Narrow::kRingU4;
 static_assert(Tiny::kRingU4 <= kLdsU4, "tiny ring exceeds the others");
 static_assert(kLdsU4 * 16 <= 160 * 1024, "LDS ring exceeds the CU's 160 KB");
@@ -411,13 +418,13 @@ __device__ __forceinline__ void stage_logits(const f32x16 (&acc)[S::kMT][S::kNT]
   const int ntok = min(S::kWT, n - r0), ne = min(S::kRows, E - c0);
   if ((ne & 7) == 0 && (dst_ld & 7) == 0 && (c0 & 7) == 0) {
     const int cpr = ne / 8;                                 // 16-byte chunks per row
-    for (int i = threadIdx.x; i < ntok * cpr; i += kThreads) {
+    for (int i = threadIdx.x; i < ntok * cpr; i += S::kNumThreads) {
       const int tl = i / cpr, c = i - tl * cpr;
       *reinterpret_cast<u32x4*>(dst + static_cast<int64_t>(row0 + r0 + tl) * dst_ld + c0 + 8 * c) =
           *reinterpret_cast<const u32x4*>(sl + tl * kStride + 8 * c);
     }
   } else {
-    for (int i = threadIdx.x; i < ntok * ne; i += kThreads) {
+    for (int i = threadIdx.x; i < ntok * ne; i += S::kNumThreads) {
       const int tl = i / ne, e = i - tl * ne;
       dst[static_cast<int64_t>(row0 + r0 + tl) * dst_ld + c0 + e] = sl[tl * kStride + e];
     }
@@ -428,7 +435,7 @@ __device__ __forceinline__ void stage_logits(const f32x16 (&acc)[S::kMT][S::kNT]
 // (i, t) of wave w, lane l lands at float (((((i * kNT + t) * 4 + q) * kWaves + w) * 64 + l) * 4
 // + v, so every store and load instruction moves 1 KB of consecutive bytes.
 template <class S>
-constexpr int kPartialFloats = S::kMT * S::kNT * 16 * kThreads;
+constexpr int kPartialFloats = S::kMT * S::kNT * 16 * S::kNumThreads;
 template <class S>
 __device__ __forceinline__ void store_partial(const f32x16 (&acc)[S::kMT][S::kNT],
                                               float* __restrict__ part) {
@@ -439,13 +446,18 @@ __device__ __forceinline__ void store_partial(const f32x16 (&acc)[S::kMT][S::kNT
     for (int t = 0; t < S::kNT; ++t)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        p[((i * S::kNT + t) * 4 + q) * kThreads] =
+        p[((i * S::kNT + t) * 4 + q) * S::kNumThreads] =
             f32x4{acc[i][t][4 * q], acc[i][t][4 * q + 1], acc[i][t][4 * q + 2], acc[i][t][4 * q + 3]};
 }
 // PARTIAL (router only): only k-tiles kt0 .. kt0 + nkt - 1 of the product, whose fp32 sums go
 // to part (store_partial) instead of logits.
+// KS > 1 (small dense and router tiles): the workgroup has KS groups of S::kNumWaves waves, each
+// with its own ring over 1 / KS of the k range; the groups' fp32 sums meet in LDS (group_sums) and
+// are added in group order, each group finishing its share of the tile.
+// DENSE: the dense MLP (dense_tiled_kernel): one group whose weights every token tile reads and
+// whose output rows the caller reads next, so neither takes the non-temporal policies.
 template <int MODE, class S, int kLdsCap = kLdsU4, bool PERSIST = false, bool STAGE = false,
-          bool PARTIAL = false>
+          bool PARTIAL = false, bool DENSE = false, int KS = 1>
 __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint16_t* __restrict__ src,
                                              int src_ld, const int32_t* __restrict__ perm_tok,
                                              int g, int r0, int n, int row0, int wt,
@@ -460,7 +472,7 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
   constexpr int kLoads = S::kLoads, kKSteps = S::kKSteps;
   constexpr int kSwzShift = S::kSwzShift;
   constexpr int kRows = S::kRows;                  // weight rows of the tile
-  static_assert(ROUTER || kRows == kWM, "expert GEMMs take kWM weight rows per tile");
+  static_assert(ROUTER || DENSE || kRows == kWM, "expert GEMMs take kWM weight rows per tile");
   static_assert(!GATEUP || kMT % 2 == 0, "gate_up pairs a wave's gate tiles with its up tiles");
   static_assert(!PARTIAL || (ROUTER && !STAGE), "partial sums are router tiles");
   const bool shared = !ROUTER && g == gw.E;
@@ -476,8 +488,12 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
   if constexpr (PERSIST) asm volatile("" : "+v"(tid));
   const int lane = tid & 63;
   // Wave index as a scalar: LDS destinations of the copies (M0) are then computed on the SALU.
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kp = KS > 1 ? wave / S::kNumWaves : 0;           // k group
+  const int w = KS > 1 ? wave - kp * S::kNumWaves : wave;
   const int wm = w % kWavesM, wn = w / kWavesM;
+  u32x4* const lds0 = lds;
+  if constexpr (KS > 1) lds += kp * S::kRingU4;
 
   // Direct global->LDS copies: wave copy i writes one contiguous 1 KB LDS block of
   // kRowsPerLoad rows; lane l fills slot l of it, i.e. row R0 + l/kChunks at swizzled position
@@ -529,13 +545,14 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
     ars[i] = raw_rsrc(base);
     aoff[i] = static_cast<uint32_t>((static_cast<int64_t>(grow) * K + 8 * j) * 2);
     if constexpr (PARTIAL) aoff[i] += static_cast<uint32_t>(kt0 * kBK * 2);
+    if constexpr (KS > 1) aoff[i] += static_cast<uint32_t>(kp * (K / KS) * 2);
   }
   // Weight bytes between k-tile kt and kt + 1 of a copy: kBK elements along the checkpoint
   // rows, or one whole k-tile block in the tiled layout (pack_tiled_kernel), where the kWM x
   // kBK k-tile is a contiguous 32 KB block in LDS order, so wave copy i reads the 1 KB at slot
   // (w * kALoads + i) * 64 of it, lane l the 16 bytes of slot l.
   int astep = kBK * 2;
-  if constexpr (!ROUTER) {
+  if constexpr (!ROUTER && !DENSE) {
     const void* tl = GATEUP ? (shared ? gw.sh_gate_up_tiled : gw.gate_up_tiled)
                             : (shared ? gw.sh_down_tiled : gw.down_tiled);
     if (tl != nullptr) {
@@ -560,6 +577,7 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
     const int srow = ROUTER ? p : (GATEUP ? (shared ? p : perm_tok[row0 + p]) : row0 + p);
     boff[i] = static_cast<uint32_t>((static_cast<int64_t>(srow) * src_ld + 8 * j) * 2);
     if constexpr (PARTIAL) boff[i] += static_cast<uint32_t>(kt0 * kBK * 2);
+    if constexpr (KS > 1) boff[i] += static_cast<uint32_t>(kp * (K / KS) * 2);
   }
 
   f32x16 acc[kMT][kNT];
@@ -575,7 +593,7 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
   // copies are non-temporal (cache policy nt), so the stream does not displace the token rows
   // and wide-tile weights that are reused (E=512 T=4096 layer 755 -> 727 us, Qwen3-30B-A3B
   // T=8192 Zipf 763 -> 741 us; the same for every tile was slower, 766 -> 799 us).
-  constexpr int kWeightPolicy = (!ROUTER && S::kWT < kWM) ? 2 : 0;
+  constexpr int kWeightPolicy = (!ROUTER && !DENSE && S::kWT < kWM) ? 2 : 0;
   // the copies of k-tile kt into ring stage `stage`
   auto issue_a = [&](int stage, int kt) {
     u32x4* buf = lds + S::a_off(stage);
@@ -606,7 +624,7 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
   // stage kt+1's first fragments and refills stage kt's buffer with k-tile kt+kStages, all
   // interleaved with the last k-step's MFMAs, so neither the copy issue nor the LDS read
   // latency of the next k-tile stands between two MFMAs.
-  const int nk = PARTIAL ? nkt : K / kBK;
+  const int nk = PARTIAL ? nkt : K / kBK / KS;
   // Wide expert tiles (MFMA-bound) put only stage 0 out before the first wait. A wave reaches
   // its wait once it has issued every copy before it, and the CU's copy path takes the waves'
   // copies in turn: with the whole ring issued up front, the second wave of each SIMD saw its
@@ -775,11 +793,74 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
 
   // Epilogue.
   const int col = lane & 31, rq = 4 * (lane >> 5);
-  if constexpr (!ROUTER) {
+  if constexpr (KS > 1) {
+    static_assert(!STAGE && !PARTIAL && !PERSIST && 4 % KS == 0, "k groups share the v4 quads");
+    constexpr int kQ = 4 / KS, kGroup = S::kNumThreads;      // quads per group, threads per group
+    constexpr int kCols = GATEUP ? kRows / 2 : kRows;        // output columns per tile
+    constexpr int kSumU4 = KS * kMT * kNT * 4 * kGroup;      // every group's accumulators
+    static_assert(kSumU4 <= KS * S::kRingU4, "the sums exceed the rings");
+    static_assert(S::kWT * (kCols / 8) <= KS * S::kRingU4, "staged tile exceeds the rings");
+    ring_barrier();                                           // every wave is done with its ring
+    f32x4* sums = reinterpret_cast<f32x4*>(lds0);
+    const int gt = w * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < kMT; ++i)
+#pragma unroll
+      for (int t = 0; t < kNT; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          sums[(((q * KS + kp) * kMT + i) * kNT + t) * kGroup + gt] =
+              f32x4{acc[i][t][4 * q], acc[i][t][4 * q + 1], acc[i][t][4 * q + 2], acc[i][t][4 * q + 3]};
+    ring_barrier();
+    f32x4 sum[kQ][kMT][kNT];
+#pragma unroll
+    for (int j = 0; j < kQ; ++j)
+#pragma unroll
+      for (int i = 0; i < kMT; ++i)
+#pragma unroll
+        for (int t = 0; t < kNT; ++t) {
+          const f32x4* p = sums + (((kp * kQ + j) * KS * kMT + i) * kNT + t) * kGroup + gt;
+          f32x4 a = p[0];
+#pragma unroll
+          for (int g2 = 1; g2 < KS; ++g2) a += p[g2 * kMT * kNT * kGroup];
+          sum[j][i][t] = a;
+        }
+    ring_barrier();                                           // the sums are read: stage the tile
+    char* st = reinterpret_cast<char*>(lds0);
+#pragma unroll
+    for (int t = 0; t < kNT; ++t) {
+      const int r = wn * (kNT * 32) + 32 * t + col;           // token within the tile
+#pragma unroll
+      for (int i = 0; i < (GATEUP ? kMT / 2 : kMT); ++i)
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+          float a[4];
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            a[v] = GATEUP ? silu(sum[j][2 * i][t][v]) * sum[j][2 * i + 1][t][v] : sum[j][i][t][v];
+          const int c = (GATEUP ? wm * (kRW / 2) : wm * kRW) + 32 * i + 8 * (kp * kQ + j) + rq;
+          *reinterpret_cast<u32x2*>(st + staged_slot<kCols>(r, c / 8) * 16 + (c % 8) * 2) =
+              u32x2{pack_bf2(a[0], a[1]), pack_bf2(a[2], a[3])};
+        }
+    }
+    ring_barrier();
+    if (!ROUTER || (c0 + kCols <= gw.E && (dst_ld & 7) == 0)) {
+      store_staged<kCols, S::kWT, false, KS * kGroup>(lds0, dst, dst_ld, row0, r0, n, c0);
+    } else {
+      // a tile past the last expert, or rows whose 16-byte chunks are not aligned
+      const uint16_t* sl = reinterpret_cast<const uint16_t*>(lds0);
+      const int ntok = min(S::kWT, n - r0), ne = min(kCols, gw.E - c0);
+      for (int i = threadIdx.x; i < ntok * ne; i += KS * kGroup) {
+        const int tl = i / ne, e = i - tl * ne;
+        dst[static_cast<int64_t>(row0 + r0 + tl) * dst_ld + c0 + e] =
+            sl[staged_slot<kCols>(tl, e / 8) * 8 + (e % 8)];
+      }
+    }
+  } else if constexpr (!ROUTER) {
     // Stage the tile in LDS as row-major [token][column] bf16, then store whole row segments
     // (kCols * 2 contiguous bytes per token) with 16-byte lanes. Storing straight from the
     // accumulators would write 16-byte pieces of 32 token rows per instruction.
-    constexpr int kCols = GATEUP ? kWM / 2 : kWM;            // output columns per tile
+    constexpr int kCols = GATEUP ? kRows / 2 : kRows;        // output columns per tile
     static_assert(S::kWT * (kCols / 8) <= kLdsCap, "staged tile exceeds the LDS ring");
     ring_barrier();                                           // every wave is done with the ring
     u32x4 next = {0xffffffffu, 0u, 0u, 0u};
@@ -823,7 +904,8 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
       }
     }
     ring_barrier();
-    store_staged<kCols, S::kWT, !GATEUP>(lds, dst, dst_ld, row0, r0, n, c0);   // down: read once
+    // the expert down's rows are read once, by the combine
+    store_staged<kCols, S::kWT, !GATEUP && !DENSE, S::kNumThreads>(lds, dst, dst_ld, row0, r0, n, c0);
   } else if constexpr (PARTIAL) {
     store_partial<S>(acc, part);
   } else if constexpr (STAGE) {
@@ -1097,6 +1179,25 @@ void tiled_persistent_kernel(GroupWeights gw, const uint16_t* __restrict__ src, 
   }
 }
 
+// The dense SwiGLU MLP (the shared expert as a module of its own), and the router logits of
+// mid-sized batches: one group of T rows, so the items are (token tile, weight tile) pairs with no
+// tile list. A few hundred tokens give few tiles, and a tile's time is then its chain of k-tiles
+// (each about 0.3 us from barrier to barrier with one or two waves per SIMD, whatever the tile),
+// not bytes or MFMAs: small tiles put a workgroup on every CU, and KS groups of waves walk 1 / KS
+// of the chain each. H = 2048, Is = 512 against the weight-streaming kernels, which reload the
+// weights for every 64 tokens: T=777 26.7 -> 15.0 us, T=8192 186 -> 50 us.
+template <int MODE, class S, int KS>
+__global__ __launch_bounds__(S::kNumThreads * KS) __attribute__((amdgpu_waves_per_eu(1)))
+void dense_tiled_kernel(GroupWeights gw, const uint16_t* __restrict__ src, int src_ld, int T,
+                        int n_wtiles, uint16_t* __restrict__ dst, int dst_ld) {
+  __shared__ u32x4 lds[S::kRingU4 * KS];
+  const int item = xcd_item(blockIdx.x, (T + S::kWT - 1) / S::kWT * n_wtiles);
+  if (item < 0) return;
+  const int ti = item / n_wtiles, wt = item - ti * n_wtiles;
+  tile_product<MODE, S, S::kRingU4, false, false, false, true, KS>(
+      gw, src, src_ld, nullptr, gw.E, ti * S::kWT, T, 0, wt, dst, dst_ld, lds);
+}
+
 // ---- host side -------------------------------------------------------------------------------
 // Upper bound of the tile-list length: rows / wide full tiles, plus per group at most one
 // partial wide tile or (wide - narrow) / narrow narrow tiles.
@@ -1259,6 +1360,68 @@ hipError_t launch_down_tiled(const GroupWeights& gw, const void* act, int act_ld
   return hipGetLastError();
 }
 
+template <int MODE, class S, int KS = 1>
+static hipError_t launch_dense_shape(const GroupWeights& gw, const void* src, int src_ld, int64_t T,
+                                     void* dst, int dst_ld, hipStream_t s) {
+  const int cols = MODE == kGateUp ? S::kRows / 2 : S::kRows;      // output columns per tile
+  const int out = MODE == kRouter ? gw.E : MODE == kGateUp ? gw.Is : gw.H;
+  const int n_wtiles = (out + cols - 1) / cols;                    // exact but for the router
+  const int64_t n_ttiles = (T + S::kWT - 1) / S::kWT;
+  dense_tiled_kernel<MODE, S, KS><<<round8(n_ttiles * n_wtiles), S::kNumThreads * KS, 0, s>>>(
+      gw, static_cast<const uint16_t*>(src), src_ld, static_cast<int>(T), n_wtiles,
+      static_cast<uint16_t*>(dst), dst_ld);
+  return hipGetLastError();
+}
+
+// 64 x 64 tiles with the k range over 4 groups of waves, or 2 where K has no 4 equal parts of
+// whole k-tiles (K is a multiple of 128).
+template <int MODE>
+static hipError_t launch_dense_small(const GroupWeights& gw, int K, const void* src, int src_ld,
+                                     int64_t T, void* dst, int dst_ld, hipStream_t s) {
+  if (K % (4 * Dense64x4::kBK) == 0)
+    return launch_dense_shape<MODE, Dense64x4, 4>(gw, src, src_ld, T, dst, dst_ld, s);
+  return launch_dense_shape<MODE, Dense64, 2>(gw, src, src_ld, T, dst, dst_ld, s);
+}
+
+// Tile of one dense GEMM (rows weight rows): the largest whose workgroups occupy most CUs, else
+// 64 x 64 with the k range split. kDenseMinWorkgroups: between the counts where a larger tile lost
+// and won. Measured (us, gate_up / down of H = 2048, Is = 512): T=777 64 x 64 in 2 k groups 9.7 /
+// 7.9 (208 / 416 workgroups), 128 x 64 12.4 / 5.4 (104 / 208); T=2048 128 x 64 13.1 / 7.2 (256 /
+// 512), 128 x 128 15.8 / 7.0 (128 / 256); T=4096 128 x 128 19.2 / 12.4, 256 x 128 23.7 / 11.4;
+// T=8192 256 x 128 31.8 / 20.0, 256 x 256 38.9 / 17.2 (128 / 256).
+template <int MODE>
+static hipError_t launch_dense_gemm(const GroupWeights& gw, const void* src, int src_ld, int64_t T,
+                                    void* dst, int dst_ld, hipStream_t s) {
+  const int rows = MODE == kGateUp ? 2 * gw.Is : gw.H, K = MODE == kGateUp ? gw.H : gw.Is;
+  auto enough = [&](int r, int t) {
+    return rows % r == 0 && (T + t - 1) / t * (rows / r) >= kDenseMinWorkgroups;
+  };
+  if (enough(Wide::kRows, Wide::kWT))
+    return launch_dense_shape<MODE, Wide>(gw, src, src_ld, T, dst, dst_ld, s);
+  if (enough(Narrow::kRows, Narrow::kWT))
+    return launch_dense_shape<MODE, Narrow>(gw, src, src_ld, T, dst, dst_ld, s);
+  if (enough(Dense128::kRows, Dense128::kWT))
+    return launch_dense_shape<MODE, Dense128>(gw, src, src_ld, T, dst, dst_ld, s);
+  if (enough(Dense128x64::kRows, Dense128x64::kWT))
+    return launch_dense_shape<MODE, Dense128x64>(gw, src, src_ld, T, dst, dst_ld, s);
+  if (enough(Dense64::kRows, Dense64::kWT))
+    return launch_dense_shape<MODE, Dense64, 2>(gw, src, src_ld, T, dst, dst_ld, s);
+  return launch_dense_small<MODE>(gw, K, src, src_ld, T, dst, dst_ld, s);
+}
+
+bool dense_tiled_supported(const GroupWeights& gw, const void* x, int64_t T, int act_ld,
+                           const void* act, const void* out) {
+  return T >= kDenseTiledMinTokens && bf16_tiled_offsets_fit(T, 0, gw.H, act_ld) &&
+         aligned16({x, act, out, gw.sh_gate, gw.sh_up, gw.sh_down});
+}
+
+hipError_t launch_dense_tiled(const GroupWeights& gw, const void* x, int64_t T, int act_ld,
+                              void* act, void* out, hipStream_t s) {
+  const hipError_t e = launch_dense_gemm<kGateUp>(gw, x, gw.H, T, act, act_ld, s);
+  if (e != hipSuccess) return e;
+  return launch_dense_gemm<kDown>(gw, act, act_ld, T, out, gw.H, s);
+}
+
 bool tiled_router_supported(int E, int H) { return H % RouterShape::kBK == 0 && E >= 1; }
 
 template <class S>
@@ -1389,12 +1552,29 @@ hipError_t launch_perm_scatter_build(const void* idx, int idx_bytes, int64_t T, 
   return hipGetLastError();
 }
 
+// Router batches in 64 x 64 tiles with the k range over four groups of waves: where the streaming
+// router would run more than kStreamRouterMaxTiles workgroups (one per 16 experts x 16 tokens;
+// past about one per CU its time grows with them, each reloading its operands), and while the
+// tiles fit the CUs at once. Measured with the selection (us, E = 512 / 128, H = 2048): T=128
+// streaming 9.2 / 8.5, these 10.8 / 10.2; T=256 12.7 / 8.7 and 10.9 / 10.2; T=777 32.3 / 10 and
+// 11.2 / 10.2; T=1024 15.4 / 14.7 (128 x 64 tiles of whole k) and 11.4 / 10.3; T=2048 16.5 / 15.0
+// and 12.9 / 10.7; T=4096 19.4 / 16.0 and 23.6 / 11.8; T=8192 30.4 / 17.9 and 42.3 / 16.2.
+constexpr int64_t kStreamRouterMaxTiles = 384;
+bool router_small_tiles(const void* x, const void* wg, const void* logits, int64_t T, int E,
+                        int H) {
+  return tiled_router_supported(E, H) && T * H * 2 < kTiledMaxBytes && aligned16({x, wg, logits}) &&
+         static_cast<int64_t>((E + 15) / 16) * ((T + 15) / 16) > kStreamRouterMaxTiles &&
+         (T + 63) / 64 * ((E + 63) / 64) <= device_cus();
+}
+
 hipError_t launch_router_logits_tiled(const void* x, const void* wg, int64_t T, int E, int H,
                                       void* logits, hipStream_t s) {
   GroupWeights gw{};
   gw.gate_up = wg;
   gw.E = E;
   gw.H = H;
+  if (router_small_tiles(x, wg, logits, T, E, H))
+    return launch_dense_small<kRouter>(gw, H, x, H, T, logits, E, s);
   if (E <= RouterShape128::kRows) return launch_router_shape<RouterShape128>(gw, x, T, logits, s);
   const int64_t tall = (T + RouterShapeTall::kWT - 1) / RouterShapeTall::kWT *
                        ((E + RouterShapeTall::kRows - 1) / RouterShapeTall::kRows);

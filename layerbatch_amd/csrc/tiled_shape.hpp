@@ -17,16 +17,19 @@ constexpr int kWaves = 8;                           // two waves per SIMD
 constexpr int kThreads = 64 * kWaves;
 constexpr int kWM = 256;                            // weight rows per workgroup
 
-// One token-tile shape: WAVES_M x (kWaves / WAVES_M) waves, each owning MT x NT units of 32
+// One token-tile shape: WAVES_M x (WAVES / WAVES_M) waves, each owning MT x NT units of 32
 // weight rows x 32 tokens, k-tiles of BK bf16 (2 * BK bytes per row), STAGES LDS buffers of
 // the weight operand and BSTAGES (STAGES or STAGES - 1) of the token operand. A symmetric ring
 // interleaves the operands per stage; an asymmetric one keeps all weight stages first. The
-// expert GEMMs use kRows = kWM weight rows; the router may use fewer.
-template <int WAVES_M, int MT, int NT, int BK, int STAGES, int BSTAGES = STAGES>
+// expert GEMMs use kRows = kWM weight rows and kWaves waves; the router and the dense MLP may use
+// fewer.
+template <int WAVES_M, int MT, int NT, int BK, int STAGES, int BSTAGES = STAGES, int WAVES = kWaves>
 struct TileShape {
+  static constexpr int kNumWaves = WAVES;
+  static constexpr int kNumThreads = 64 * WAVES;
   static constexpr int kRows = WAVES_M * MT * 32;             // weight rows per workgroup
   static constexpr int kWavesM = WAVES_M;
-  static constexpr int kWavesN = kWaves / WAVES_M;
+  static constexpr int kWavesN = WAVES / WAVES_M;
   static constexpr int kMT = MT;
   static constexpr int kNT = NT;
   static constexpr int kRW = MT * 32;                         // weight rows per wave
@@ -36,8 +39,8 @@ struct TileShape {
   static constexpr int kBStages = BSTAGES;
   static constexpr int kChunks = BK / 8;                      // 16-byte chunks per LDS row
   static constexpr int kRowsPerLoad = 64 / kChunks;           // rows one wave copy covers
-  static constexpr int kALoads = kRows / kRowsPerLoad / kWaves;  // wave copies per stage (weights)
-  static constexpr int kBLoads = kWT / kRowsPerLoad / kWaves;  // wave copies per stage (tokens)
+  static constexpr int kALoads = kRows / kRowsPerLoad / WAVES;  // wave copies per stage (weights)
+  static constexpr int kBLoads = kWT / kRowsPerLoad / WAVES;  // wave copies per stage (tokens)
   static constexpr int kLoads = kALoads + kBLoads;
   static constexpr int kStageU4 = (kRows + kWT) * kChunks;    // 16-byte slots per stage
   static constexpr int kAU4 = kRows * kChunks, kBU4 = kWT * kChunks;
@@ -51,7 +54,7 @@ struct TileShape {
   // kChunks: 16 consecutive rows then hit 16 distinct 16-byte bank groups for any fixed j.
   static constexpr int kSwzShift = kChunks == 4 ? 2 : 1;
   static_assert(kChunks == 4 || kChunks == 8, "BK must be 32 or 64");
-  static_assert(kALoads * kRowsPerLoad * kWaves == kRows && kBLoads * kRowsPerLoad * kWaves == kWT,
+  static_assert(kALoads * kRowsPerLoad * WAVES == kRows && kBLoads * kRowsPerLoad * WAVES == kWT,
                 "copies must tile the stage");
   static_assert(kKSteps % 2 == 0, "the next k-tile's first fragments go to register buffer 0");
   static __device__ __forceinline__ int swz(int r, int j) {
@@ -101,11 +104,11 @@ __device__ __forceinline__ int staged_slot(int r, int c) {
 // 16-byte lanes, whole row segments at a time. NT: non-temporal stores, for output that only
 // the combine reads back once (the down GEMMs: E=512 T=4096 down 256 -> 245 us, fp8 E=512
 // T=16384 413 -> 405 us), so that it does not displace the operands the GEMM reuses.
-template <int kCols, int kTokens, bool NT = false>
+template <int kCols, int kTokens, bool NT = false, int kBlock = kThreads>
 __device__ __forceinline__ void store_staged(const u32x4* __restrict__ st, uint16_t* __restrict__ dst,
                                              int dst_ld, int row0, int r0, int n, int c0) {
   constexpr int kRowChunks = kCols / 8;
-  constexpr int kRowsPerPass = kThreads / kRowChunks;
+  constexpr int kRowsPerPass = kBlock / kRowChunks;
   const int c = threadIdx.x % kRowChunks;
   for (int r = threadIdx.x / kRowChunks; r < kTokens; r += kRowsPerPass) {
     const int p = r0 + r;
