@@ -69,7 +69,12 @@ _SIGS = {
 }
 
 EXPORTED = tuple(_SIGS)
+# the entry points that the host extension calls, in the order of its table
+_HOST_FNS = ("lbmoe_status_string", "lbmoe_workspace_size", "lbmoe_forward", "lbmoe_forward_norm",
+             "lbmoe_router_logits", "lbmoe_route", "lbmoe_experts",
+             "lbmoe_dense_mlp_workspace_size", "lbmoe_dense_mlp")
 _lib = None
+_host = None
 
 
 def lib():
@@ -86,6 +91,23 @@ def lib():
             fn.argtypes = args
         _lib = h
     return _lib
+
+
+def host(classes):
+    """The host extension (csrc/host_ext.cpp), bound to the library and to the module classes
+    (router, experts, shared-expert MLP, block)."""
+    global _host
+    if _host is None:
+        h = lib()
+        try:
+            from . import _host as ext
+        except ImportError as e:
+            raise RuntimeError(f"the host extension does not load ({e}): build it with "
+                               "`python -m layerbatch_amd.build`") from e
+        ext.bind(tuple(ctypes.cast(getattr(h, n), _p).value for n in _HOST_FNS),
+                 (*classes, torch.nn.Linear))
+        _host = ext
+    return _host
 
 
 def check(status, what):

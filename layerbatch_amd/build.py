@@ -1,20 +1,23 @@
-"""Build liblbmoe.so (gfx950) in-tree with hipcc.
+"""Build liblbmoe.so (gfx950) and the host extension in-tree.
 
-    python -m layerbatch_amd.build          # compile every csrc/*.hip, link liblbmoe.so
+    python -m layerbatch_amd.build   # compile every csrc/*.hip, link liblbmoe.so; build _host.so
 
-Objects go to layerbatch_amd/_build/, the library to layerbatch_amd/liblbmoe.so. The HIP code
-is compiled with packed-fp32 instruction generation disabled.
+Objects go to layerbatch_amd/_build/, the library to layerbatch_amd/liblbmoe.so (hipcc, with
+packed-fp32 instruction generation disabled), the CPython extension of csrc/host_ext.cpp, which
+uses torch's C++ tensors, to layerbatch_amd/_host.so (the host compiler).
 """
 import concurrent.futures as cf
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "liblbmoe.so")
+HOST = os.path.join(PKG, "_host.so")
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -45,13 +48,37 @@ def _compile(hipcc, src):
     return obj, warn
 
 
+def _build_host():
+    """Compile and link the host extension against the installed torch."""
+    import torch
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("no host C++ compiler found (set CXX)")
+    root = os.path.dirname(torch.__file__)
+    inc, rocm = os.path.join(root, "include"), os.environ.get("ROCM_PATH", "/opt/rocm")
+    tmp = HOST + ".tmp"
+    cmd = [cxx, "-O2", "-fPIC", "-std=c++17", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I" + inc, "-I" + os.path.join(inc, "torch", "csrc", "api", "include"),
+           "-I" + os.path.join(rocm, "include"), "-I" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "host_ext.cpp"), "-o", tmp, "-L" + os.path.join(root, "lib"),
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"host extension build failed:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, HOST)
+
+
 def build(verbose=False):
-    """Compile all sources and link liblbmoe.so. Returns the library path."""
+    """Compile all sources, link liblbmoe.so and build the host extension. Returns the library
+    path."""
     hipcc = _hipcc()
     os.makedirs(BUILD, exist_ok=True)
     srcs = sources()
-    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        host = ex.submit(_build_host)
         results = list(ex.map(lambda s: _compile(hipcc, s), srcs))
+        host.result()
     for obj, warn in results:
         if warn and verbose:
             print(warn, file=sys.stderr)

@@ -27,6 +27,10 @@ and decoder layer (qwen3_5.py:956-962, :1004) use them unchanged. Differences, a
   residual add, post_attention_layernorm and the block in one call (qwen3_5.py:998-1004),
   returning (block output, new residual).
 
+Every forward first offers the call to the host extension (csrc/host_ext.cpp), which runs the plain
+case natively and returns None for anything it does not take, refused calls included; the Python
+code after it is the general path, with every check and its message.
+
 Every forward runs on the tensor's CUDA (HIP) device on the current stream, enqueues HIP
 kernels only (no host synchronisation), and raises RuntimeError for CPU tensors, wrong dtypes
 or a missing library build.
@@ -42,6 +46,11 @@ from ._lib import LbmoeLayer, check, lib, ptr
 
 __all__ = ["Qwen3_5TopKRouter", "Qwen3_5Experts", "Qwen3_5SharedExpertMLP",
            "Qwen3_5SparseMoeBlock"]
+
+
+def _host():
+    return _lib._host or _lib.host((Qwen3_5TopKRouter, Qwen3_5Experts, Qwen3_5SharedExpertMLP,
+                                    Qwen3_5SparseMoeBlock))
 
 
 def _require(t, name, dtype=torch.bfloat16, ndim=None):
@@ -148,6 +157,9 @@ class Qwen3_5TopKRouter(nn.Module):
         return out
 
     def forward(self, hidden_states: torch.Tensor):
+        out = _host().router(self, hidden_states)
+        if out is not None:
+            return out
         logits = self.logits(hidden_states)
         T = hidden_states.shape[0]
         dev = hidden_states.device
@@ -225,6 +237,9 @@ class Qwen3_5Experts(nn.Module):
                 L.down_tiled = self.down_tiled.data_ptr()
 
     def forward(self, hidden_states, top_k_indices, top_k_weights):
+        out = _host().experts(self, hidden_states, top_k_indices, top_k_weights)
+        if out is not None:
+            return out
         _require(hidden_states, "hidden_states", ndim=2)
         _require(top_k_indices, "top_k_indices", None, 2)
         _require(top_k_weights, "top_k_weights", torch.bfloat16, 2)
@@ -291,6 +306,9 @@ class Qwen3_5SharedExpertMLP(nn.Module):
             L.shared_down_tiled = self.down_tiled.data_ptr()
 
     def forward(self, x):
+        out = _host().mlp(self, x)
+        if out is not None:
+            return out
         _require(x, "x", ndim=2)
         _same_device(self, x.device)
         T, H = x.shape
@@ -368,6 +386,9 @@ class Qwen3_5SparseMoeBlock(nn.Module):
         return _lib.workspace_size(self.layer(), T)
 
     def forward(self, hidden_states: torch.Tensor, workspace: torch.Tensor = None):
+        out = _host().block(self, hidden_states, workspace)
+        if out is not None:
+            return out
         _require(hidden_states, "hidden_states", ndim=2)
         _require_width(hidden_states, self.experts.hidden_size)
         _same_device(self, hidden_states.device)
@@ -392,6 +413,9 @@ class Qwen3_5SparseMoeBlock(nn.Module):
         norm is the layer's post_attention_layernorm (a Qwen3_5RMSNorm: ``weight`` [H] and
         ``eps``). Returns (block output, new residual); the inputs are not modified.
         """
+        out = _host().block_norm(self, hidden_states, residual, norm, workspace)
+        if out is not None:
+            return out
         _require(hidden_states, "hidden_states", ndim=2)
         _require(residual, "residual", ndim=2)
         _require(norm.weight, "norm.weight", ndim=1)
