@@ -222,7 +222,12 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
   } else if (!permuted && !perm_in_gate_up) {
     const bool tiled = use_tiled(gw, T, k) &&
                        (!is_fp8(L) || tiled_fp8_supported(gw, T, T * k + (with_shared ? T : 0)));
-    if (tiled && perm_chunked(T * k, E)) {
+    if (tiled && perm_build_supported(T * k, T, max_tiles)) {
+      LBMOE_TRY(launch_perm_build(idx, idx_bytes, T, k, counts, offsets, perm_tok,
+                                  at<int32_t>(ws, w, R_PERM_SLOT), inv, gw, with_shared, max_tiles,
+                                  tiles, s));
+      tiles_built = true;
+    } else if (tiled && perm_chunked(T * k, E)) {
       // prefill GEMMs: the permutation's scatter and the tile list in one launch
       int32_t* base = at<int32_t>(ws, w, R_BASE);
       int32_t* lrank = at<int32_t>(ws, w, R_LRANK);

@@ -312,6 +312,13 @@ hipError_t launch_perm_scatter_build(const void* idx, int idx_bytes, int64_t T, 
                                      const int32_t* lrank, int32_t* offsets, int32_t* perm_tok,
                                      int32_t* perm_slot, int32_t* inv, const GroupWeights& gw,
                                      bool shared, int max_tiles, int32_t* tiles, hipStream_t s);
+// The whole permutation of at most kPermBuildEntries entries and the tile list in one launch.
+constexpr int kPermBuildEntries = 8192;
+bool perm_build_supported(int64_t V, int64_t T, int max_tiles);
+hipError_t launch_perm_build(const void* idx, int idx_bytes, int64_t T, int k, int32_t* counts,
+                             int32_t* offsets, int32_t* perm_tok, int32_t* perm_slot, int32_t* inv,
+                             const GroupWeights& gw, bool shared, int max_tiles, int32_t* tiles,
+                             hipStream_t s);
 hipError_t launch_scatter_build(const int32_t* idx, int64_t T, int k, const int32_t* base,
                                 const int32_t* counts, const int32_t* lrank, int32_t* offsets,
                                 int32_t* perm_tok, int32_t* perm_slot, int32_t* inv,

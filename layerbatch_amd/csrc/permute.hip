@@ -18,6 +18,7 @@
 // Entries whose expert id lies outside [0, E) are left out of every list and get inv = -1.
 #include "common.hpp"
 #include "internal.hpp"
+#include "perm_single.hpp"
 #include "route_token.hpp"
 
 namespace lbmoe {
@@ -218,105 +219,14 @@ __global__ __launch_bounds__(64) void perm_scatter(const void* idx, int T, int k
   }
 }
 
-// Whole permutation in one workgroup for decode-sized batches (V <= R * kPermSingle): thread
-// tid takes entries v = r * kPermSingle + tid, r < R, so that "virtual wave" vw = v / 64 =
-// r * (kPermSingle / 64) + wave covers 64 consecutive entries. Each virtual wave ranks its
-// entries among equal experts (ballot match) and records its count per expert; one thread per
-// expert then turns the counts into per-virtual-wave prefixes (in v order) and a total, a block
-// scan of the totals gives the offsets, and every entry lands at offsets[e] + (entries of e in
-// earlier virtual waves) + rank.
-// The body, for a workgroup of kPermSingle threads that all call it (idx may point to LDS).
-template <int IB, int R, int EMAX>
-__device__ __forceinline__ void perm_single_body(const void* idx, int T, int k, int E, int nbits,
-                                                 int V, int32_t* counts, int32_t* offsets,
-                                                 int32_t* perm_tok, int32_t* perm_slot,
-                                                 int32_t* inv) {
-  constexpr int kW = kPermSingle / kWave;
-  constexpr int kVW = kW * R;            // virtual waves
-  __shared__ int cnt[kVW][EMAX];         // per virtual wave and expert: count, then prefix
-  __shared__ int start[EMAX];
-  __shared__ int wsum[kW];
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-  for (int i = tid; i < kVW * EMAX; i += kPermSingle) (&cnt[0][0])[i] = 0;
-  int e[R], s[R], t[R], rank[R];
-  bool valid[R];
-  // unconditional loads (entries past V read entry V-1 and are masked); V = 0 reads nothing
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    e[r] = -1;
-    s[r] = t[r] = 0;
-  }
-  if (V > 0) {                           // the same for every thread
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int v = min(r * kPermSingle + tid, V - 1);
-      s[r] = v / T;
-      t[r] = v - s[r] * T;
-      e[r] = load_expert<IB>(idx, static_cast<int64_t>(t[r]) * k + s[r]);
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (r * kPermSingle + tid >= V) e[r] = -1;
-  }
-  uint64_t m[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    valid[r] = (e[r] >= 0) && (e[r] < E);
-    m[r] = match_expert(valid[r] ? e[r] : 0, __ballot(valid[r]), nbits);
-    rank[r] = mask_rank(m[r]);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-    if (valid[r] && rank[r] == 0) cnt[r * kW + wave][e[r]] = __popcll(m[r]);
-  __syncthreads();
-  int total = 0;
-  if (tid < E) {
-    for (int w = 0; w < kVW; ++w) {
-      const int c = cnt[w][tid];
-      cnt[w][tid] = total;
-      total += c;
-    }
-  }
-  int incl = total;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const int y = __shfl_up(incl, o, kWave);
-    if (lane >= o) incl += y;
-  }
-  if (lane == kWave - 1) wsum[wave] = incl;
-  __syncthreads();
-  int before = 0;
-  for (int w = 0; w < wave; ++w) before += wsum[w];
-  const int excl = before + incl - total;
-  if (tid < E) {
-    start[tid] = excl;
-    counts[tid] = total;
-    offsets[tid] = excl;
-  }
-  if (tid == kPermSingle - 1) offsets[E] = before + incl;
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (r * kPermSingle + tid >= V) continue;
-    const int64_t ts = static_cast<int64_t>(t[r]) * k + s[r];
-    if (!valid[r]) {
-      inv[ts] = -1;
-    } else {
-      const int pos = start[e[r]] + cnt[r * kW + wave][e[r]] + rank[r];
-      perm_tok[pos] = t[r];
-      perm_slot[pos] = s[r];
-      inv[ts] = pos;
-    }
-  }
-}
-
 template <int IB, int R, int EMAX>
 __global__ __launch_bounds__(kPermSingle) void perm_single(const void* idx, int T, int k, int E,
                                                            int nbits, int V, int32_t* counts,
                                                            int32_t* offsets, int32_t* perm_tok,
                                                            int32_t* perm_slot, int32_t* inv) {
-  perm_single_body<IB, R, EMAX>(idx, T, k, E, nbits, V, counts, offsets, perm_tok, perm_slot, inv);
+  __shared__ PermSingleLds<R, EMAX> lds;
+  perm_single_body<IB, R, EMAX>(lds, idx, T, k, E, nbits, V, counts, offsets, perm_tok, perm_slot,
+                                inv);
 }
 
 // Route and permutation of a small batch (route_perm_small_supported) in one workgroup: wave t selects token t's experts (route_token), the indices go
@@ -335,8 +245,10 @@ __global__ __launch_bounds__(kPermSingle) void route_perm_small(
   __syncthreads();
   const int V = T * k;
   if (static_cast<int>(threadIdx.x) < V) idx[threadIdx.x] = s_idx[threadIdx.x];
-  perm_single_body<4, 1, 1024>(s_idx, T, k, E, nbits, V, counts, offsets, perm_tok, perm_slot,
-                               inv);
+  constexpr int kEMax = EPL <= 2 ? 128 : EPL * kWave;       // EPL * 64 >= E
+  __shared__ PermSingleLds<1, kEMax> lds;
+  perm_single_body<4, 1, kEMax>(lds, s_idx, T, k, E, nbits, V, counts, offsets, perm_tok, perm_slot,
+                                inv);
 }
 
 __global__ __launch_bounds__(256) void fill_i32_kernel(int32_t* p, int64_t n, int32_t value) {
@@ -370,9 +282,16 @@ static hipError_t launch_permute_t(const void* idx, int64_t T, int k, int E, int
                                                        counts, offsets, perm_tok, perm_slot, inv);
     return hipGetLastError();
   };
-  if (V <= kPermSingle) return single.template operator()<1, 1024>();
-  if (V <= 2 * kPermSingle) return single.template operator()<2, 1024>();
-  if (V <= 4 * kPermSingle && E <= 512) return single.template operator()<4, 512>();
+  auto by_experts = [&]<int R>() {
+    if (E <= 128) return single.template operator()<R, 128>();
+    if (E <= 256) return single.template operator()<R, 256>();
+    if (E <= 512) return single.template operator()<R, 512>();
+    if constexpr (R <= 2) return single.template operator()<R, 1024>();
+    else return hipErrorInvalidValue;                       // not reached
+  };
+  if (V <= kPermSingle) return by_experts.template operator()<1>();
+  if (V <= 2 * kPermSingle) return by_experts.template operator()<2>();
+  if (V <= 4 * kPermSingle && E <= 512) return by_experts.template operator()<4>();
   // hist, base: E x nblk; lrank: V; the per-expert totals are the counts
   const int nblk = static_cast<int>(perm_blocks(V));
   perm_count<IB><<<nblk, 64, 0, s>>>(idx, static_cast<int>(T), k, E, nbits, V, nblk, hist,

@@ -139,9 +139,17 @@ __device__ __forceinline__ int dispatch_item(int b, int W, int N) {
   const int tail = min(nn, kTailSlots);
   const int spread = nn - tail, prefix = nw + spread;
   if (j >= prefix) return W + n0 + spread + (j - prefix);       // the tail: narrow items
-  // narrow items before slot j in the prefix: floor(j * spread / prefix)
-  const int before = static_cast<int>(static_cast<int64_t>(j) * spread / prefix);
-  const int upto = static_cast<int>(static_cast<int64_t>(j + 1) * spread / prefix);
+  // narrow items before slot j in the prefix: floor(j * spread / prefix). In 32 bits where the
+  // product fits (a 64-bit division is some 150 instructions, two per entry)
+  int before, upto;
+  if (prefix < 65536) {
+    const uint32_t p = prefix, m = static_cast<uint32_t>(j) * spread;
+    before = static_cast<int>(m / p);
+    upto = static_cast<int>((m + spread) / p);
+  } else {
+    before = static_cast<int>(static_cast<int64_t>(j) * spread / prefix);
+    upto = static_cast<int>(static_cast<int64_t>(j + 1) * spread / prefix);
+  }
   return upto > before ? W + n0 + before : w0 + (j - before);
 }
 
@@ -365,6 +373,95 @@ __global__ __launch_bounds__(1024) void perm_scatter_build_kernel(
   perm_tok[pos] = t;
   perm_slot[pos] = s;
   inv[ts] = pos;
+}
+
+// The whole permutation of a batch of at most R * 1024 entries and the tile list in one launch.
+// Workgroup b places the entries of experts [b * 2^ebits, (b + 1) * 2^ebits) and writes its share of
+// the dispatch tables (build_tiles_body). Every workgroup reads all V ids (from L2) and counts all
+// experts with LDS atomics, whose order does not matter, for the experts' first rows; it ranks only
+// its own experts' entries: thread tid takes entries v = r * 1024 + tid, so that virtual wave
+// r * 16 + wave covers 64 consecutive entries of the (slot, token) order, lanes of equal experts rank
+// by ballot match on the low ebits bits, and one wave per own expert turns the per-virtual-wave
+// counts into prefixes. t_magic = ceil(2^32 / T): v / T without a division (exact for v < 2^16).
+// Bound by latency, so one launch whose workgroups repeat the cheap counting beats perm_single (one
+// CU: 12-16 us for 4072 ids) and build_tiles_kernel (6 us) after it, or for more entries the count,
+// scan and scatter launches (18 us): E = 128, 4072 entries 20 -> 9 us, the experts call 231 -> 222 us;
+// with a one-workgroup form of this kernel 14-17 us.
+constexpr int kPermBuildBlocks = 64;
+template <int IB, int R>
+__global__ __launch_bounds__(1024) void perm_build_kernel(
+    const void* idx, int T, int k, uint32_t t_magic, int E, int ebits, int V, int32_t* counts,
+    int32_t* offsets, int32_t* perm_tok, int32_t* perm_slot, int32_t* inv, int shared, int sh_row0,
+    int max_tiles, int wide, int narrow, int tiny, int I, int Is, int H, int grid_gu, int grid_dn,
+    int32_t* __restrict__ tiles) {
+  constexpr int kVW = 16 * R;                              // virtual waves
+  constexpr int kOwn = 1024 / kPermBuildBlocks;            // own experts at most
+  static_assert(kVW % 64 == 0 || kVW < 64, "a wave scans 64 virtual waves at a time");
+  __shared__ int total[1024], start[1024], cnt[kOwn][kVW], wsum[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int e[R], s[R], t[R], rank[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int v = min(r * 1024 + tid, V - 1);              // unconditional loads, V >= 1
+    s[r] = static_cast<int>(__umulhi(static_cast<uint32_t>(v), t_magic));
+    t[r] = v - s[r] * T;
+    e[r] = load_expert<IB>(idx, static_cast<int64_t>(t[r]) * k + s[r]);
+  }
+  total[tid] = 0;
+  for (int i = tid; i < kOwn * kVW; i += 1024) (&cnt[0][0])[i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool valid = r * 1024 + tid < V && e[r] >= 0 && e[r] < E;
+    if (valid) atomicAdd(&total[e[r]], 1);
+    const bool own = valid && (e[r] >> ebits) == static_cast<int>(blockIdx.x);
+    const uint64_t m = match_expert(own ? e[r] : 0, __ballot(own), ebits);
+    rank[r] = own ? mask_rank(m) : -1;
+    if (rank[r] == 0) cnt[e[r] & ((1 << ebits) - 1)][r * 16 + wave] = __popcll(m);
+  }
+  __syncthreads();
+  int ex;
+  const int all = block_scan_1024(total[tid], ex, wsum);   // total is 0 from E on
+  start[tid] = ex;
+  if (blockIdx.x == 0) {
+    if (tid < E) {
+      counts[tid] = total[tid];
+      offsets[tid] = ex;
+    }
+    if (tid == 0) offsets[E] = all;
+  }
+  if (wave < (1 << ebits)) {                               // at most kOwn = 16 waves
+    int before = 0;
+#pragma unroll
+    for (int c = 0; c < (kVW + 63) / 64; ++c) {
+      const int vw = c * 64 + lane;
+      const int n = vw < kVW ? cnt[wave][vw] : 0;
+      int incl = n;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o, kWave);
+        if (lane >= o) incl += y;
+      }
+      if (vw < kVW) cnt[wave][vw] = before + incl - n;
+      before += __shfl(incl, 63, kWave);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (r * 1024 + tid >= V) continue;
+    const int64_t ts = static_cast<int64_t>(t[r]) * k + s[r];
+    if (rank[r] >= 0) {
+      const int pos = start[e[r]] + cnt[e[r] & ((1 << ebits) - 1)][r * 16 + wave] + rank[r];
+      perm_tok[pos] = t[r];
+      perm_slot[pos] = s[r];
+      inv[ts] = pos;
+    } else if (blockIdx.x == 0 && (e[r] < 0 || e[r] >= E)) {
+      inv[ts] = -1;
+    }
+  }
+  build_tiles_body(total, start, E, shared, T, sh_row0, max_tiles, wide, narrow, tiny, I, Is, H,
+                   grid_gu, grid_dn, tiles, blockIdx.x, gridDim.x);
 }
 
 // ---- one token tile --------------------------------------------------------------------------
@@ -1565,6 +1662,36 @@ bool router_small_tiles(const void* x, const void* wg, const void* logits, int64
   return tiled_router_supported(E, H) && T * H * 2 < kTiledMaxBytes && aligned16({x, wg, logits}) &&
          static_cast<int64_t>((E + 15) / 16) * ((T + 15) / 16) > kStreamRouterMaxTiles &&
          (T + 63) / 64 * ((E + 63) / 64) <= device_cus();
+}
+
+bool perm_build_supported(int64_t V, int64_t T, int max_tiles) {
+  return V >= 1 && V <= kPermBuildEntries && T >= 2 && max_tiles <= kLdsListEntries;
+}
+
+hipError_t launch_perm_build(const void* idx, int idx_bytes, int64_t T, int k, int32_t* counts,
+                             int32_t* offsets, int32_t* perm_tok, int32_t* perm_slot, int32_t* inv,
+                             const GroupWeights& gw, bool shared, int max_tiles, int32_t* tiles,
+                             hipStream_t s) {
+  const int V = static_cast<int>(T * k);
+  int ebits = 2;                              // 4 own experts, more where E needs it
+  while (((gw.E - 1) >> ebits) >= kPermBuildBlocks) ++ebits;
+  const int blocks = ((gw.E - 1) >> ebits) + 1;
+  const auto magic = static_cast<uint32_t>(((uint64_t{1} << 32) + T - 1) / T);
+  const int grid_gu = tiled_grid(gw, max_tiles, true), grid_dn = tiled_grid(gw, max_tiles, false);
+  auto run = [&]<int IB, int R>() {
+    perm_build_kernel<IB, R><<<blocks, 1024, 0, s>>>(
+        idx, static_cast<int>(T), k, magic, gw.E, ebits, V, counts, offsets, perm_tok, perm_slot,
+        inv, shared ? 1 : 0, gw.sh_row0, max_tiles, Wide::kWT, Narrow::kWT, Tiny::kWT, gw.I, gw.Is,
+        gw.H, grid_gu, grid_dn, tiles);
+    return hipGetLastError();
+  };
+  auto by_entries = [&]<int IB>() {
+    if (V <= 2 * 1024) return run.template operator()<IB, 2>();
+    if (V <= 4 * 1024) return run.template operator()<IB, 4>();
+    return run.template operator()<IB, 8>();
+  };
+  static_assert(kPermBuildEntries == 8 * 1024, "entries of the largest kernel");
+  return idx_bytes == 8 ? by_entries.template operator()<8>() : by_entries.template operator()<4>();
 }
 
 hipError_t launch_router_logits_tiled(const void* x, const void* wg, int64_t T, int E, int H,

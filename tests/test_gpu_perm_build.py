@@ -1,0 +1,65 @@
+"""The permutation with the tile list in one launch (batches of at most 8192 routing pairs on the
+LDS-tiled GEMMs) against the CPU oracle."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from layerbatch_amd import _lib
+from layerbatch_amd.synth import MoEShape, make_layer, make_x
+from oracle import moe as om
+from tests import gpu_checks as gc
+from tests.helpers import layer_np, to_np
+from tests.test_gpu_parity import _block
+
+pytestmark = pytest.mark.gpu
+
+
+# 2 / 4 / 8 entries per thread and one entry past each, the last size of all (8192) and the chunked
+# permutation after it; 2 to 1000 experts (4 to 16 per workgroup); ids outside [0, E)
+@pytest.mark.parametrize("T,k,E,dt", [
+    (1024, 2, 8, torch.int64), (683, 3, 20, torch.int32), (2048, 2, 48, torch.int32),
+    (4097, 1, 3, torch.int64), (1024, 8, 128, torch.int64), (1639, 5, 256, torch.int32),
+    (800, 10, 300, torch.int64), (1000, 8, 1000, torch.int32), (57, 2, 2, torch.int32)])
+def test_experts_perm_build(gpu, T, k, E, dt):
+    shape = MoEShape(256, E, k, 256 if E >= 300 else 128, 0)
+    w, g = make_layer(shape, seed=T)
+    x = make_x(g, T, 256)
+    blk = _block(shape, {n: v.to(gpu) for n, v in w.items()}, gpu)
+    rng = np.random.default_rng(T)
+    idx = np.argsort(rng.random((T, E)), axis=1)[:, :k].astype(np.int64)
+    idx[3, 0], idx[T - 1, k - 1] = E, -1                   # dropped pairs
+    tw = (torch.rand((T, k), generator=g) + 0.1).to(torch.bfloat16)
+    d_idx, d_tw, xd = torch.from_numpy(idx).to(gpu, dt), tw.to(gpu), x.to(gpu)
+    L = _lib.LbmoeLayer()
+    blk.experts.fill_layer(L)
+    L.top_k = k
+    y = torch.empty_like(xd)
+    ws = torch.empty(_lib.workspace_size(L, T), dtype=torch.uint8, device=gpu)
+    _lib.check(_lib.lib().lbmoe_experts(
+        ctypes.byref(L), _lib.ptr(xd), _lib.ptr(d_idx), d_idx.element_size(), _lib.ptr(d_tw), T,
+        _lib.ptr(y), _lib.ptr(ws), ws.numel(), _lib.stream_of(gpu)), "lbmoe_experts")
+    torch.cuda.synchronize()
+
+    def region(name, n):
+        off, _ = _lib.workspace_region(L, T, name)
+        return ws[off:off + 4 * n].view(torch.int32).cpu().numpy()
+
+    # the oracle's order of the kept pairs: expert, then slot, then token
+    key = [(idx[t, s], s, t) for s in range(k) for t in range(T) if 0 <= idx[t, s] < E]
+    key.sort(key=lambda v: v[0])                            # stable: (slot, token) within an expert
+    n = len(key)
+    np.testing.assert_array_equal(region("counts", E), np.bincount([v[0] for v in key], minlength=E))
+    np.testing.assert_array_equal(region("perm_slot", n), [v[1] for v in key])
+    np.testing.assert_array_equal(region("perm_tok", n), [v[2] for v in key])
+    inv = np.full((T, k), -1)
+    for r, (_, s, t) in enumerate(key):
+        inv[t, s] = r
+    np.testing.assert_array_equal(region("inv", T * k).reshape(T, k), inv)
+    ok = (idx >= 0) & (idx < E)
+    wn = layer_np(w)
+    rows = rng.choice(T, 24, replace=False) if T > 24 else np.arange(T)
+    ref = om.experts(to_np(x)[rows], np.where(ok, idx, 0)[rows], np.where(ok, to_np(tw), 0.0)[rows],
+                     wn["gate_up"], wn["down"])
+    gc.check_output(to_np(y)[rows], ref, gc.TOL_BF16)
