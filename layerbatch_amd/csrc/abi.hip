@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstring>
 
 #include "internal.hpp"
@@ -158,16 +159,38 @@ static P* at(void* ws, const WsLayout& w, int r) {
     if ((expr) != hipSuccess) return LBMOE_ERR_LAUNCH;        \
   } while (0)
 
-// Expected tokens per routed expert at which the LDS-tiled GEMMs replace weight streaming.
-// Measured (back-to-back µs per layer call): at 24 tokens per expert both are even
-// (Qwen3-30B-A3B T=384: 286-291); from 30 on the tiled GEMMs win clearly (T=512: 293 vs 431,
-// E=512 T=1536: 731 vs 998), the streaming kernels then needing four token tiles per pass;
-// at 20 streaming wins (E=512 T=1024: 672 vs 714, fp8 427 vs 484).
-constexpr double kTiledMinTokensPerExpert = 28.0;
+// Expected tokens per routed expert from which the LDS-tiled GEMMs replace weight streaming. The
+// streaming kernels run two token tiles per pass above 8 tokens per expert and four above 28, each
+// step slower; the tiled ones barely depend on the count, but their items (one per expert and 128
+// intermediate channels at these sizes) must fill whole rounds of the CUs. Measured (GPU us per layer
+// call, streaming / tiled):
+//   bf16, 8 items per CU (E = 512, I = 512): 7.5 tokens per expert 535 / 531, 20 tokens 639 / 565
+//   bf16, 3 (E = 128, I = 768): 12 tokens 211 / 222, 16 tokens 225 / 223, 24 tokens 257 / 230
+//   bf16, 2.25 and 1.5 (0.75 of the last round's CUs or less busy): 16 tokens 184 / 209 and 73 / 72,
+//     24 tokens 218 / 209 and 91 / 77; 1.17: 23 tokens 117 / 134
+//   fp8 (its streaming kernels stream less per wave): 10 tokens 339 / 328 (8 items per CU) and 82 /
+//     81 (2), 12 tokens 149 / 129 (3) and 61 / 50 (0.75)
+// Below 0.7 items per CU the tiled launches leave CUs idle and only the four-tile passes are slower
+// (E = 16, I = 512: 25 tokens 32 / 36). Skewed routings gain more: under a Zipf bias the streaming
+// kernels walk a popular expert's rows pass after pass (E = 512, 7.5 tokens: 477 / 139).
+// Below kTiledAlways only operands on 16-byte boundaries (of the copies) leave the streaming kernels.
+constexpr double kTiledAlways = 28.0;
+static double tiled_min_tokens(const GroupWeights& gw, bool fp8) {
+  const double n = static_cast<double>(gw.E) * (gw.I / 128) / device_cus();   // items per CU
+  const double full = n / std::ceil(n);
+  if (fp8) return n >= 0.7 ? 10.0 : kTiledAlways;
+  if (n >= 4.0) return 8.0;
+  if (n >= 1.0 && full >= 0.9) return 16.0;
+  return full >= 0.7 ? 24.0 : kTiledAlways;
+}
 
-static bool use_tiled(const GroupWeights& gw, int64_t T, int k) {
-  return tiled_supported(gw) && tiled_offsets_fit(gw, T, k) &&
-         static_cast<double>(T) * k / gw.E >= kTiledMinTokensPerExpert;
+static bool use_tiled(const lbmoe_layer& L, const GroupWeights& gw, const void* x, int64_t T,
+                      int k) {
+  if (!tiled_supported(gw) || !tiled_offsets_fit(gw, T, k)) return false;
+  const double avg = static_cast<double>(T) * k / gw.E;
+  if (avg >= kTiledAlways) return true;
+  return avg >= tiled_min_tokens(gw, is_fp8(L)) &&
+         aligned16({x, gw.gate_up, gw.down, gw.sh_gate, gw.sh_up, gw.sh_down});
 }
 
 // Routed experts of one call: permute, gate_up, down, combine.
@@ -206,7 +229,7 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
   if (T * k < E) gw.hit_rows = static_cast<int>(T * k);
   // the route's own ids (all in [0, E)) can be permuted inside the bf16 decode gate_up kernel
   const bool perm_in_gate_up = own_ids && !permuted && idx_bytes == 4 && !is_fp8(L) &&
-                               !use_tiled(gw, T, k) && gate_up_perm_supported(gw, T, k);
+                               !use_tiled(L, gw, x, T, k) && gate_up_perm_supported(gw, T, k);
   int32_t* tiles = at<int32_t>(ws, w, R_TILES);
   const int max_tiles = tiled_max_tiles(T * k + (with_shared ? T : 0), gw.groups);
   bool tiles_built = false;
@@ -220,7 +243,7 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
                                    max_tiles, tiles, s));
     tiles_built = true;
   } else if (!permuted && !perm_in_gate_up) {
-    const bool tiled = use_tiled(gw, T, k) &&
+    const bool tiled = use_tiled(L, gw, x, T, k) &&
                        (!is_fp8(L) || tiled_fp8_supported(gw, T, T * k + (with_shared ? T : 0)));
     if (tiled && perm_build_supported(T * k, T, max_tiles)) {
       LBMOE_TRY(launch_perm_build(idx, idx_bytes, T, k, counts, offsets, perm_tok,
@@ -254,7 +277,7 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
     float* acts = at<float>(ws, w, R_ACTS);
     const int64_t rows = T * k + (with_shared ? T : 0);
     if (!x_quantised) LBMOE_TRY(launch_quant_groups_fp8(x, T, H, H, xq, xs, s));
-    if (use_tiled(gw, T, k) && tiled_fp8_supported(gw, T, rows)) {
+    if (use_tiled(L, gw, x, T, k) && tiled_fp8_supported(gw, T, rows)) {
       if (!tiles_built)
         LBMOE_TRY(launch_build_tiles(counts, offsets, gw, with_shared, T, max_tiles, tiles, s));
       LBMOE_TRY(launch_gate_up_tiled_fp8(gw, xq, xs, perm_tok, tiles, max_tiles, Imax, actq, acts,
@@ -272,8 +295,8 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
     LBMOE_TRY(ev->mark(s));
     return LBMOE_OK;
   }
-  if (rt && use_tiled(gw, T, k)) return LBMOE_ERR_SHAPE;   // not reached (see forward_impl)
-  if (use_tiled(gw, T, k)) {
+  if (rt && use_tiled(L, gw, x, T, k)) return LBMOE_ERR_SHAPE;   // not reached (see forward_impl)
+  if (use_tiled(L, gw, x, T, k)) {
     // prefill-sized batch: LDS-tiled MFMA GEMMs over a device-built token-tile list
     if (!tiles_built)
       LBMOE_TRY(launch_build_tiles(counts, offsets, gw, with_shared, T, max_tiles, tiles, s));
@@ -410,11 +433,11 @@ struct NormArgs {
 
 // Whether the block routes through launch_router_route: the tiled router over at most 128
 // experts, with the tiled expert GEMMs after it (their tile list is built with the scatter).
-static bool route_in_router(const lbmoe_layer& L, int64_t T, bool sh) {
+static bool route_in_router(const lbmoe_layer& L, const void* x, int64_t T, bool sh) {
   const int E = L.num_experts, H = L.hidden_size, k = L.top_k;
   if (!router_is_tiled(T, E, H) || !router_route_supported(E, H, k)) return false;
   const GroupWeights gw = group_weights(L, sh, T);
-  if (!use_tiled(gw, T, k)) return false;
+  if (!use_tiled(L, gw, x, T, k)) return false;
   return !is_fp8(L) || tiled_fp8_supported(gw, T, T * k + (sh ? T : 0));
 }
 
@@ -438,7 +461,7 @@ static int32_t forward_impl(const lbmoe_layer* layer, const void* x, int64_t T, 
   void* topw = at<void>(ws, w, R_TOPW);
   float* sgate = sh ? at<float>(ws, w, R_SGATE) : nullptr;
   LBMOE_TRY(ev->mark(s));
-  if (!norm && route_in_router(L, T, sh)) {
+  if (!norm && route_in_router(L, x, T, sh)) {
     // logits, selection and the permutation's count pass in one launch, or two with the k range
     // split (profiled calls time it as the router stage, the routing stage then being empty);
     // the split's partial sums go to the expert-output region, which only the down GEMM writes

@@ -1,5 +1,5 @@
 """The permutation with the tile list in one launch (batches of at most 8192 routing pairs on the
-LDS-tiled GEMMs) against the CPU oracle."""
+LDS-tiled GEMMs), and the token counts per expert where those GEMMs begin, against the CPU oracle."""
 import ctypes
 
 import numpy as np
@@ -11,7 +11,7 @@ from layerbatch_amd.synth import MoEShape, make_layer, make_x
 from oracle import moe as om
 from tests import gpu_checks as gc
 from tests.helpers import layer_np, to_np
-from tests.test_gpu_parity import _block
+from tests.test_gpu_parity import _block, _run_and_check
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +63,27 @@ def test_experts_perm_build(gpu, T, k, E, dt):
     ref = om.experts(to_np(x)[rows], np.where(ok, idx, 0)[rows], np.where(ok, to_np(tw), 0.0)[rows],
                      wn["gate_up"], wn["down"])
     gc.check_output(to_np(y)[rows], ref, gc.TOL_BF16)
+
+
+# tokens per expert on either side of the switch: 8 items per CU, whole rounds, partly filled ones
+@pytest.mark.parametrize("shape,T", [
+    (MoEShape(256, 512, 2, 512, 128), 2047), (MoEShape(256, 512, 2, 512, 128), 2048),
+    (MoEShape(256, 256, 4, 256, 0), 1023), (MoEShape(256, 256, 4, 256, 0), 1024),
+    (MoEShape(256, 96, 2, 512, 128), 1151), (MoEShape(256, 96, 2, 512, 128), 1152)])
+def test_block_at_the_switch(gpu, shape, T):
+    _run_and_check(shape, T, gpu, seed=T, sample=48)
+
+
+def test_unaligned_rows_at_the_switch(gpu):
+    """Token rows between 16-byte boundaries: the same result (below 28 tokens per expert they stay
+    on the streaming kernels)."""
+    shape, T = MoEShape(256, 256, 4, 256, 0), 1024
+    w, g = make_layer(shape, seed=4)
+    blk = _block(shape, {n: v.to(gpu) for n, v in w.items()}, gpu)
+    xd = make_x(g, T, 256).to(gpu)
+    view = torch.empty(T * 256 + 1, dtype=torch.bfloat16, device=gpu)[1:].view(T, 256)
+    view.copy_(xd)
+    a, b = to_np(blk(xd)).astype("float64"), to_np(blk(view)).astype("float64")
+    # a router logit summed in another order may move a token to another expert: all but a few rows
+    close = np.abs(a - b).max(axis=1) <= gc.TOL_BF16 * np.abs(a).max()
+    assert close.mean() >= 0.99
