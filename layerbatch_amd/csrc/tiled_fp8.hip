@@ -26,17 +26,26 @@ namespace f8t {
 
 // The LDS ring of 128-byte k-tiles (TileShape counts k-tiles in bf16 units: BK = 64).
 using Wide = TileShape<2, 4, 2, 64, 2>;
-using Narrow = TileShape<2, 4, 1, 64, 2>;
+using Narrow = TileShape<4, 2, 2, 64, 3>;     // 4 x 2 waves of 64 x 64: 128 tokens
 using Tiny = TileShape<4, 2, 1, 64, 3>;       // 4 x 2 waves of 64 x 32: 64 tokens
-constexpr int kRingU4 = Wide::kStages * Wide::kStageU4;
-static_assert(Narrow::kStages * Narrow::kStageU4 <= kRingU4, "narrow ring exceeds the wide one");
-static_assert(Tiny::kStages * Tiny::kStageU4 <= kRingU4, "tiny ring exceeds the wide one");
 // Scale blocks per row (K / 128) the LDS scale area holds: K <= 3072.
 constexpr int kMaxKBlocks = 24;
-constexpr int kActScales = kMaxKBlocks * Wide::kWT;
 constexpr int kWScales = 64;                  // two rows of kMaxKBlocks, copied by one wave
 static_assert(2 * kMaxKBlocks <= kWScales, "weight-scale rows exceed one wave copy");
-static_assert(kRingU4 * 16 + (kActScales + kWScales) * 4 <= 160 * 1024, "LDS exceeds 160 KB");
+// One LDS object: a shape's ring, behind it the activation scales of its tokens and the two
+// weight-scale rows; the persistent kernel's next entry and queue state in the last 32 bytes.
+constexpr int kLdsU4 = 160 * 1024 / 16;
+template <class S> constexpr int kShapeRingU4 = S::kStages * S::kStageU4;
+template <class S> constexpr int kActScales = kMaxKBlocks * S::kWT;
+template <class S>
+constexpr bool kFits = kShapeRingU4<S> * 16 + (kActScales<S> + kWScales) * 4 + 32 <= kLdsU4 * 16;
+static_assert(kFits<Wide> && kFits<Narrow> && kFits<Tiny>, "LDS exceeds 160 KB");
+
+// Position of 16-byte chunk j of LDS row r: j ^ chunk_xor(r). A fragment read takes chunks 2q and
+// 2q + 1 of 16 consecutive rows (q = lane / 16); under this XOR a ds_read_b128's lanes hit distinct
+// banks (an LDS probe over eight row functions), where the bf16 reads' XOR, (r / 2) mod 8, leaves
+// them two-way conflicted.
+__device__ __forceinline__ int chunk_xor(int r) { return ((r & 3) << 1) | ((r >> 2) & 1); }
 
 __device__ __forceinline__ i32x8 cat8(u32x4 lo, u32x4 hi) {
   return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
@@ -61,7 +70,7 @@ __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
                                                  int r0, int n, int row0, int wt,
                                                  void* __restrict__ dst, int dst_ld,
                                                  float* __restrict__ dst_sc,
-                                                 u32x4* __restrict__ lds, float* __restrict__ scl) {
+                                                 u32x4* __restrict__ lds) {
   constexpr int kM16 = 2 * S::kMT;               // 16-row tiles per wave
   constexpr int kN16 = 2 * S::kNT;               // 16-token tiles per wave
   constexpr int kRW = S::kRW, kWT = S::kWT, kWavesM = S::kWavesM;
@@ -69,6 +78,7 @@ __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
   constexpr int kALoads = S::kALoads, kBLoads = S::kBLoads, kLoads = S::kLoads;
   constexpr int kStageU4 = S::kStageU4;
   static_assert(kChunks == 8, "a k-tile is 128 bytes per row");
+  float* scl = reinterpret_cast<float*>(lds + kShapeRingU4<S>);
   const bool shared = g == gw.E;
   const int Ig = shared ? gw.Is : gw.I;
   const int H = gw.H;
@@ -127,7 +137,7 @@ __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
   for (int i = 0; i < kALoads; ++i) {
     const int row0c = (w * kALoads + i) * kRowsPerLoad;        // the copy's first row
     const int row = row0c + lrow;
-    const int j = lpos ^ ((row >> S::kSwzShift) & (kChunks - 1));
+    const int j = lpos ^ chunk_xor(row);
     if (GATEUP) {
       const int half = row0c / kRW, sub0 = row0c % kRW;
       abase[i] = sub0 < kRW / 2 ? wbase : wup;
@@ -146,7 +156,7 @@ __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
   for (int i = 0; i < kBLoads; ++i) {
     const int lt = (w * kBLoads + i) * kRowsPerLoad + lrow;
     const int row = kWM + lt;
-    const int j = lpos ^ ((row >> S::kSwzShift) & (kChunks - 1));
+    const int j = lpos ^ chunk_xor(row);
     boff[i] = static_cast<uint32_t>(src_row(lt)) * static_cast<uint32_t>(src_ld) + 16 * j;
   }
 
@@ -168,10 +178,10 @@ __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
     }
     if (w == 0) {
       const float* wsp = lane < nk ? sw0 + lane : (lane < 2 * nk ? sw1 + (lane - nk) : sw0);
-      __builtin_amdgcn_global_load_lds(wsp, (lds_ptr)(scl + kActScales), 4, 0, 0);
+      __builtin_amdgcn_global_load_lds(wsp, (lds_ptr)(scl + kActScales<S>), 4, 0, 0);
     }
   }
-  const float* wsc = scl + kActScales;
+  const float* wsc = scl + kActScales<S>;
 
   f32x4 acc[kM16][kN16];
 #pragma unroll
@@ -200,13 +210,17 @@ __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
   };
 
   const int r16 = lane & 15, q = lane >> 4;
+  auto read_row = [&](const u32x4* buf, int row) {
+    const int x = chunk_xor(row);
+    return cat8(buf[row * kChunks + ((2 * q) ^ x)], buf[row * kChunks + ((2 * q + 1) ^ x)]);
+  };
   auto read_a = [&](const u32x4* buf, int i) {
     const int row = wm * kRW + 16 * i + r16;
-    return cat8(buf[S::swz(row, 2 * q)], buf[S::swz(row, 2 * q + 1)]);
+    return read_row(buf, row);
   };
   auto read_b = [&](const u32x4* buf, int t) {
     const int row = kWM + wn * (16 * kN16) + 16 * t + r16;
-    return cat8(buf[S::swz(row, 2 * q)], buf[S::swz(row, 2 * q + 1)]);
+    return read_row(buf, row);
   };
   // Ring protocol of the bf16 kernels: all kStages buffers are filled up front; in k-tile kt,
   // once the last A tile's fragments are in registers, each wave waits for its copies of
@@ -321,7 +335,7 @@ __device__ __forceinline__ void tile_product_fp8(const GroupWeights& gw,
 
   // Epilogue: stage the tile in the ring as [token][column] bf16, then store row segments.
   constexpr int kCols = GATEUP ? kWM / 2 : kWM;
-  static_assert(kWT * (kCols / 8) <= kRingU4, "staged tile exceeds the LDS ring");
+  static_assert(kWT * (kCols / 8) <= kShapeRingU4<S>, "staged tile exceeds the LDS ring");
   ring_barrier();                                           // every wave is done with the ring
   char* st = reinterpret_cast<char*>(lds);
 #pragma unroll
@@ -373,19 +387,18 @@ void tiled_fp8_kernel(GroupWeights gw, const uint8_t* __restrict__ src,
                       const float* __restrict__ src_sc, int src_ld,
                       const int32_t* __restrict__ perm_tok, const u32x4* __restrict__ table,
                       void* __restrict__ dst, int dst_ld, float* __restrict__ dst_sc) {
-  __shared__ u32x4 lds[kRingU4];
-  __shared__ float scl[kActScales + kWScales];
+  __shared__ u32x4 lds[kLdsU4];
   const TileItem it = decode_item(table[blockIdx.x]);
   if (it.g < 0) return;
   if (it.tiny)
     tile_product_fp8<GATEUP, Tiny>(gw, src, src_sc, src_ld, perm_tok, it.g, it.r0, it.n,
-                                   it.row0, it.wt, dst, dst_ld, dst_sc, lds, scl);
+                                   it.row0, it.wt, dst, dst_ld, dst_sc, lds);
   else if (it.narrow)
     tile_product_fp8<GATEUP, Narrow>(gw, src, src_sc, src_ld, perm_tok, it.g, it.r0, it.n,
-                                     it.row0, it.wt, dst, dst_ld, dst_sc, lds, scl);
+                                     it.row0, it.wt, dst, dst_ld, dst_sc, lds);
   else
     tile_product_fp8<GATEUP, Wide>(gw, src, src_sc, src_ld, perm_tok, it.g, it.r0, it.n,
-                                   it.row0, it.wt, dst, dst_ld, dst_sc, lds, scl);
+                                   it.row0, it.wt, dst, dst_ld, dst_sc, lds);
 }
 
 // gate_up as one workgroup per CU taking entries from the per-XCD work queues of the dispatch
@@ -397,29 +410,29 @@ void tiled_fp8_persistent_kernel(GroupWeights gw, const uint8_t* __restrict__ sr
                                  const int32_t* __restrict__ perm_tok,
                                  const u32x4* __restrict__ table, int slots, int* __restrict__ q,
                                  void* __restrict__ dst, int dst_ld, float* __restrict__ dst_sc) {
-  __shared__ u32x4 lds[kRingU4];
-  __shared__ float scl[kActScales + kWScales];
-  __shared__ u32x4 ent;
-  __shared__ int tried;                // the queue state lives in LDS, not across the loop
-  if (threadIdx.x == 0) tried = 0;
+  __shared__ u32x4 lds[kLdsU4];
+  // the next entry and the queue state live in LDS, not across the loop
+  u32x4& ent = lds[kLdsU4 - 1];
+  u32x4& state = lds[kLdsU4 - 2];
+  if (threadIdx.x == 0) state[0] = 0;
   for (;;) {
     if (threadIdx.x == 0) {
-      WorkQueue wq{table, slots, q, static_cast<int>(blockIdx.x & 7), tried, 0};
+      WorkQueue wq{table, slots, q, static_cast<int>(blockIdx.x & 7), static_cast<int>(state[0]), 0};
       ent = queue_fetch(wq);
-      tried = wq.tried;
+      state[0] = static_cast<uint32_t>(wq.tried);
     }
     __syncthreads();
     const TileItem it = decode_item(ent);
     if (it.g < 0) break;               // the same for the whole workgroup
     if (it.tiny)
       tile_product_fp8<true, Tiny, true>(gw, src, src_sc, src_ld, perm_tok, it.g, it.r0, it.n,
-                                         it.row0, it.wt, dst, dst_ld, dst_sc, lds, scl);
+                                         it.row0, it.wt, dst, dst_ld, dst_sc, lds);
     else if (it.narrow)
       tile_product_fp8<true, Narrow, true>(gw, src, src_sc, src_ld, perm_tok, it.g, it.r0, it.n,
-                                           it.row0, it.wt, dst, dst_ld, dst_sc, lds, scl);
+                                           it.row0, it.wt, dst, dst_ld, dst_sc, lds);
     else
       tile_product_fp8<true, Wide, true>(gw, src, src_sc, src_ld, perm_tok, it.g, it.r0, it.n,
-                                         it.row0, it.wt, dst, dst_ld, dst_sc, lds, scl);
+                                         it.row0, it.wt, dst, dst_ld, dst_sc, lds);
   }
 }
 
@@ -431,13 +444,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 void dense_tiled_fp8_kernel(GroupWeights gw, const uint8_t* __restrict__ src,
                             const float* __restrict__ src_sc, int src_ld, int T, int n_wtiles,
                             void* __restrict__ dst, int dst_ld, float* __restrict__ dst_sc) {
-  __shared__ u32x4 lds[kRingU4];
-  __shared__ float scl[kActScales + kWScales];
+  __shared__ u32x4 lds[kLdsU4];
   const int item = xcd_item(blockIdx.x, (T + S::kWT - 1) / S::kWT * n_wtiles);
   if (item < 0) return;
   const int ti = item / n_wtiles, wt = item - ti * n_wtiles;
   tile_product_fp8<GATEUP, S, false, true>(gw, src, src_sc, src_ld, nullptr, gw.E, ti * S::kWT, T,
-                                           0, wt, dst, dst_ld, dst_sc, lds, scl);
+                                           0, wt, dst, dst_ld, dst_sc, lds);
 }
 
 template <bool GATEUP, class S>
