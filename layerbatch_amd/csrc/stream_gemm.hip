@@ -679,8 +679,14 @@ __device__ __forceinline__ int inline_route(const GroupWeights& gw, const SmallR
   return s_res[0];
 }
 
-template <int MAXB, int EPL>
-__global__ __launch_bounds__(64 * kSplitMaxWaves) void gate_up_bf16_routed_kernel(
+// MINW: waves per SIMD that the register allocation keeps room for. Left to itself (2) the compiler
+// takes 130 VGPRs for more loads ahead, which holds three workgroups per CU; with 4 it takes 116 and
+// four workgroups fit (Qwen3-30B-A3B T=4 58.1 -> 56.8 us per layer, T=5 73.5 with three -> 67.8; E =
+// 64, I = 512, T=5, 3.75 workgroups per CU: 30.9 -> 27.5), but with about three per CU or fewer the
+// loads ahead are worth more (E = 32, I = 768, T=4, 3.2: 34.8 against 37.0).
+template <int MAXB, int EPL, int MINW>
+__global__ __launch_bounds__(64 * kSplitMaxWaves)
+__attribute__((amdgpu_waves_per_eu(MINW))) void gate_up_bf16_routed_kernel(
     GroupWeights gw, const uint16_t* __restrict__ x, SmallRoute rt, int T, int shared_extra,
     int act_ld, uint16_t* __restrict__ act) {
   __shared__ int toks[kInlineRouteTokens];
@@ -734,8 +740,17 @@ hipError_t launch_gate_up_bf16_routed(const GroupWeights& gw, const void* x, con
   auto* a = static_cast<uint16_t*>(act);
   const int Ti = static_cast<int>(T);
   return with_maxb<1>(plan, [&]<int TT_, int MAXB>() {
-#define LBMOE_ROUTED(EPL) \
-  gate_up_bf16_routed_kernel<MAXB, EPL><<<grid, 64 * plan.waves, 0, s>>>(gw, xx, rt, Ti, extra, act_ld, a)
+  // EPL = 16 does not fit four waves per SIMD
+  const bool four = static_cast<int64_t>(grid.x) * grid.y * 2 > 7 * device_cus();
+#define LBMOE_ROUTED(EPL)                                                                         \
+  do {                                                                                            \
+    if (four && EPL <= 8)                                                                         \
+      gate_up_bf16_routed_kernel<MAXB, EPL, EPL <= 8 ? 4 : 2>                                     \
+          <<<grid, 64 * plan.waves, 0, s>>>(gw, xx, rt, Ti, extra, act_ld, a);                    \
+    else                                                                                          \
+      gate_up_bf16_routed_kernel<MAXB, EPL, 2>                                                    \
+          <<<grid, 64 * plan.waves, 0, s>>>(gw, xx, rt, Ti, extra, act_ld, a);                    \
+  } while (0)
     if (gw.E <= 64) LBMOE_ROUTED(1);
     else if (gw.E <= 128) LBMOE_ROUTED(2);
     else if (gw.E <= 256) LBMOE_ROUTED(4);
