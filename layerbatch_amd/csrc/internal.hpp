@@ -127,6 +127,10 @@ inline int shared_extra_rows(const GroupWeights& gw, int64_t T, int tokens_per_p
 // ---- launchers (each returns hipError_t of the launch) ----------------------------------
 hipError_t launch_router_logits(const void* x, const void* wg, int64_t T, int E, int H,
                                 void* logits, hipStream_t s);
+// Residual add + RMSNorm of the decoder layer ahead of the block: x_out = the block's input, res_out
+// = the new residual.
+hipError_t launch_add_rmsnorm(const void* hidden, const void* residual, const void* norm_w, float eps,
+                              int64_t T, int H, void* x_out, void* res_out, hipStream_t s);
 // Residual add + RMSNorm of the decoder layer ahead of the block, then the router logits of
 // its output: x_out = the block's input, res_out = the new residual (fused into the router
 // for decode-sized T).

@@ -320,6 +320,15 @@ hipError_t launch_router_logits(const void* x, const void* wg, int64_t T, int E,
 // T=512 431 vs 422).
 constexpr int64_t kNormFusedMaxTokens = 16;
 
+hipError_t launch_add_rmsnorm(const void* hidden, const void* residual, const void* norm_w, float eps,
+                              int64_t T, int H, void* x_out, void* res_out, hipStream_t s) {
+  add_rmsnorm_kernel<<<static_cast<unsigned>((T + 3) / 4), 256, 0, s>>>(
+      static_cast<const uint16_t*>(hidden), static_cast<const uint16_t*>(residual),
+      static_cast<const uint16_t*>(norm_w), eps, static_cast<int>(T), H,
+      static_cast<uint16_t*>(x_out), static_cast<uint16_t*>(res_out));
+  return hipGetLastError();
+}
+
 hipError_t launch_add_rmsnorm_router(const void* hidden, const void* residual, const void* norm_w,
                                      float eps, const void* wg, int64_t T, int E, int H,
                                      void* logits, void* x_out, void* res_out, hipStream_t s) {
@@ -329,9 +338,7 @@ hipError_t launch_add_rmsnorm_router(const void* hidden, const void* residual, c
   const int per_wave = (H / kKBlock + kRouterWaves - 1) / kRouterWaves;
   if (T <= kNormFusedMaxTokens && per_wave <= kRouterNormBlocks)
     return launch_router_decode<true>(nullptr, nm, wg, T, E, H, logits, s);
-  add_rmsnorm_kernel<<<static_cast<unsigned>((T + 3) / 4), 256, 0, s>>>(
-      nm.hidden, nm.residual, nm.weight, eps, static_cast<int>(T), H, nm.x_out, nm.res_out);
-  const hipError_t e = hipGetLastError();
+  const hipError_t e = launch_add_rmsnorm(hidden, residual, norm_w, eps, T, H, x_out, res_out, s);
   if (e != hipSuccess) return e;
   return launch_router_logits(x_out, wg, T, E, H, logits, s);
 }
