@@ -691,6 +691,23 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
   // and wide-tile weights that are reused (E=512 T=4096 layer 755 -> 727 us, Qwen3-30B-A3B
   // T=8192 Zipf 763 -> 741 us; the same for every tile was slower, 766 -> 799 us).
   constexpr int kWeightPolicy = (!ROUTER && !DENSE && S::kWT < kWM) ? 2 : 0;
+  const int nk = PARTIAL ? nkt : K / kBK / KS;
+  // Narrow and tiny tiles walk the k range from a start of their own (the group's and weight tile's,
+  // so the sums do not depend on timing). From k = 0 together, the workgroups in flight read the same
+  // 128 bytes of every 4 KB row at about the same time, which lands on few HBM channels, how few
+  // depending on where the weights were allocated: Qwen3-30B-A3B experts T=509 221-254 us by
+  // allocation, rotated 209; T=512 layer 235-266 -> 220, T=2048 333-345 -> 322, E=512 T=4096 703 ->
+  // 692. Wide tiles stay in step: they share operands through L2 (T=8192 uniform 744 -> 768 us
+  // rotated), and the fp8 tiles, with half the bytes per row, gain nothing (E=512 T=4096 477 -> 480).
+  constexpr bool kRotate = !ROUTER && !DENSE && S::kWT < kWM;
+  const int rot = kRotate ? static_cast<int>((5u * static_cast<uint32_t>(wt) + 3u * static_cast<uint32_t>(g)) %
+                                             static_cast<uint32_t>(nk))
+                          : 0;
+  auto k_of = [&](int kt) {                   // k-tile of the matrix at step kt of the product
+    if constexpr (!kRotate) return kt;
+    const int r = kt + rot;
+    return r >= nk ? r - nk : r;
+  };
   // the copies of k-tile kt into ring stage `stage`
   auto issue_a = [&](int stage, int kt) {
     u32x4* buf = lds + S::a_off(stage);
@@ -698,7 +715,7 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
     for (int i = 0; i < kALoads; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           ars[i], (lds_ptr)(buf + (w * kALoads + i) * kRowsPerLoad * kChunks), 16, aoff[i],
-          kt * astep, 0, kWeightPolicy);
+          k_of(kt) * astep, 0, kWeightPolicy);
   };
   auto issue_b = [&](int stage, int kt) {
     u32x4* buf = lds + S::b_off(stage);
@@ -706,7 +723,7 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
     for (int i = 0; i < kBLoads; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           brs, (lds_ptr)(buf + ((w * kBLoads + i) * kRowsPerLoad) * kChunks), 16, boff[i],
-          kt * (kBK * 2), 0, 0);
+          k_of(kt) * (kBK * 2), 0, 0);
   };
   auto issue = [&](int stage, int kt) {
     issue_a(stage, kt);
@@ -721,7 +738,6 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
   // stage kt+1's first fragments and refills stage kt's buffer with k-tile kt+kStages, all
   // interleaved with the last k-step's MFMAs, so neither the copy issue nor the LDS read
   // latency of the next k-tile stands between two MFMAs.
-  const int nk = PARTIAL ? nkt : K / kBK / KS;
   // Wide expert tiles (MFMA-bound) put only stage 0 out before the first wait. A wave reaches
   // its wait once it has issued every copy before it, and the CU's copy path takes the waves'
   // copies in turn: with the whole ring issued up front, the second wave of each SIMD saw its
