@@ -165,9 +165,11 @@ static P* at(void* ws, const WsLayout& w, int r) {
 // intermediate channels at these sizes) must fill whole rounds of the CUs. Measured (GPU us per layer
 // call, streaming / tiled):
 //   bf16, 8 items per CU (E = 512, I = 512): 7.5 tokens per expert 535 / 531, 20 tokens 639 / 565
-//   bf16, 3 (E = 128, I = 768): 12 tokens 211 / 222, 16 tokens 225 / 223, 24 tokens 257 / 230
-//   bf16, 2.25 and 1.5 (0.75 of the last round's CUs or less busy): 16 tokens 184 / 209 and 73 / 72,
-//     24 tokens 218 / 209 and 91 / 77; 1.17: 23 tokens 117 / 134
+//   bf16, 3 and 2, whole rounds (E = 128, I = 768; E = 256, I = 256): 10 tokens 204 / 207 and 104 /
+//     106, 14 tokens 218 / 209 and 111 / 109
+//   bf16, 2.25 and 1.5 (the last round three quarters full or less): 12 tokens 173 / 183 and 113 / 117,
+//     20 tokens 197 / 186 and 126 / 120; 0.75: 17 tokens 80 / 79
+//   bf16, 1.17 and 1.25: 15 tokens 103 / 118 and 70 / 73, 27 tokens 137 / 123
 //   fp8 (its streaming kernels stream less per wave): 10 tokens 339 / 328 (8 items per CU) and 82 /
 //     81 (2), 12 tokens 149 / 129 (3) and 61 / 50 (0.75)
 // Below 0.7 items per CU the tiled launches leave CUs idle and only the four-tile passes are slower
@@ -180,8 +182,9 @@ static double tiled_min_tokens(const GroupWeights& gw, bool fp8) {
   const double full = n / std::ceil(n);
   if (fp8) return n >= 0.7 ? 10.0 : kTiledAlways;
   if (n >= 4.0) return 8.0;
-  if (n >= 1.0 && full >= 0.9) return 16.0;
-  return full >= 0.7 ? 24.0 : kTiledAlways;
+  if (full >= 0.9 && n >= 1.0) return 13.0;
+  if (full >= 0.7) return 17.0;
+  return n >= 1.0 ? 24.0 : kTiledAlways;
 }
 
 static bool use_tiled(const lbmoe_layer& L, const GroupWeights& gw, const void* x, int64_t T,

@@ -68,8 +68,8 @@ def test_experts_perm_build(gpu, T, k, E, dt):
 # tokens per expert on either side of the switch: 8 items per CU, whole rounds, partly filled ones
 @pytest.mark.parametrize("shape,T", [
     (MoEShape(256, 512, 2, 512, 128), 2047), (MoEShape(256, 512, 2, 512, 128), 2048),
-    (MoEShape(256, 256, 4, 256, 0), 1023), (MoEShape(256, 256, 4, 256, 0), 1024),
-    (MoEShape(256, 96, 2, 512, 128), 1151), (MoEShape(256, 96, 2, 512, 128), 1152)])
+    (MoEShape(256, 256, 4, 256, 0), 831), (MoEShape(256, 256, 4, 256, 0), 832),
+    (MoEShape(256, 96, 2, 512, 128), 815), (MoEShape(256, 96, 2, 512, 128), 816)])
 def test_block_at_the_switch(gpu, shape, T):
     _run_and_check(shape, T, gpu, seed=T, sample=48)
 
