@@ -497,10 +497,11 @@ static int32_t forward_impl(const lbmoe_layer* layer, const void* x, int64_t T, 
     LBMOE_TRY(launch_router_logits(x, L.gate_weight, T, L.num_experts, L.hidden_size, logits, s));
   }
   LBMOE_TRY(ev->mark(s));
+  const GroupWeights gw = group_weights(L, sh, T);
+  const bool streams = !is_fp8(L) && !use_tiled(L, gw, x, T, L.top_k);   // the bf16 decode GEMMs
   // the smallest bf16 batches route inside the gate_up kernel (profiled calls then have
-  // empty routing and permutation stages; T*k/E <= 4 tokens per expert never reaches the
-  // tiled GEMMs)
-  if (!is_fp8(L) && inline_route_supported(T, L.top_k, L.num_experts)) {
+  // empty routing and permutation stages)
+  if (streams && inline_route_supported(T, L.top_k, L.num_experts)) {
     const SmallRoute rt{static_cast<const uint16_t*>(logits), L.logit_bias,
                         static_cast<const uint16_t*>(L.shared_expert_gate), L.top_k,
                         static_cast<int32_t*>(idx), static_cast<uint16_t*>(topw), sgate,
@@ -514,9 +515,7 @@ static int32_t forward_impl(const lbmoe_layer* layer, const void* x, int64_t T, 
   // stage, their permutation stage then being empty), unless the gate_up kernel permutes: the
   // selection spread over CUs then is shorter (Qwen3-30B-A3B T=16 128.6 -> 126.9 us, E = 16 T=8
   // 22.8 -> 21.9 us)
-  const GroupWeights gw = group_weights(L, sh, T);
-  const bool perm_in_gate_up = !is_fp8(L) && T * L.top_k >= L.num_experts &&
-                               !use_tiled(L, gw, x, T, L.top_k) &&
+  const bool perm_in_gate_up = streams && T * L.top_k >= L.num_experts &&
                                gate_up_perm_supported(gw, T, L.top_k);
   if (!perm_in_gate_up && route_perm_small_supported(T, L.top_k, L.num_experts)) {
     LBMOE_TRY(launch_route_perm_small(
