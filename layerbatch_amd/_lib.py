@@ -100,12 +100,13 @@ def host(classes):
     if _host is None:
         h = lib()
         try:
+            from torch.utils._device import DeviceContext
             from . import _host as ext
         except ImportError as e:
             raise RuntimeError(f"the host extension does not load ({e}): build it with "
                                "`python -m layerbatch_amd.build`") from e
         ext.bind(tuple(ctypes.cast(getattr(h, n), _p).value for n in _HOST_FNS),
-                 (*classes, torch.nn.Linear))
+                 (*classes, torch.nn.Linear, DeviceContext))
         _host = ext
     return _host
 

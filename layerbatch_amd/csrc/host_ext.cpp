@@ -8,9 +8,10 @@
 // them anew.
 //
 // Each entry takes the plain case only: modules and tensors of exactly the expected types, with the
-// attributes that moe.py's constructors and load_fp8_ leave, no packed weights, no torch modes or
-// transforms in effect. It returns None for anything else (a wrong shape, dtype or device included)
-// before any allocation or launch, and moe.py's general path then runs the call or raises.
+// attributes that moe.py's constructors and load_fp8_ leave, no packed weights, no torch modes (but a
+// default device) or transforms in effect. It returns None for anything else (a wrong shape, dtype
+// or device included) before any allocation or launch, and moe.py's general path then runs the call
+// or raises.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -20,6 +21,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/utils/pybind.h>
@@ -45,8 +47,8 @@ struct Abi {
 };
 Abi abi{};
 
-// The module classes, set by bind (strong references).
-PyTypeObject *t_router, *t_experts, *t_mlp, *t_block, *t_linear;
+// The module classes and torch's default-device mode, set by bind (strong references).
+PyTypeObject *t_router, *t_experts, *t_mlp, *t_block, *t_linear, *t_device_context;
 
 struct Names {
   PyObject *parameters, *modules, *weight, *bias, *gate, *experts, *shared_expert,
@@ -114,11 +116,15 @@ struct Tensors {
   }
 };
 
-// Torch function or dispatch modes, functorch transforms: the general path's business.
+// Torch function or dispatch modes, functorch transforms: the general path's business. A default
+// device is let through: torch.set_default_device leaves its mode on the stack for good (an engine's
+// model runner sets one), and it only gives a device to calls that name none, which no allocation
+// here or in the general path is.
 bool plain_torch() {
-  if (at::impl::PythonTorchFunctionTLS::stack_len() > 0 ||
-      c10::impl::TorchDispatchModeTLS::any_modes_set())
-    return false;
+  using Modes = at::impl::PythonTorchFunctionTLS;
+  for (int64_t i = 0, n = Modes::stack_len(); i < n; ++i)
+    if (Py_TYPE(Modes::get_stack_at(i)->ptr(getPyInterpreter())) != t_device_context) return false;
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
   constexpr c10::DispatchKeySet special({c10::DispatchKey::Python,
                                          c10::DispatchKey::PythonTLSSnapshot,
                                          c10::DispatchKey::Functionalize,
@@ -438,12 +444,21 @@ PyObject* mlp(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// Whether the modes and transforms in effect leave a call to this extension.
+PyObject* plain(PyObject*, PyObject*) {
+  HANDLE_TH_ERRORS
+  return PyBool_FromLong(plain_torch());
+  END_HANDLE_TH_ERRORS
+}
+
 // bind(addresses, classes): addresses of the entry points in Abi's order; (router, experts, mlp,
-// block, nn.Linear) classes.
+// block, nn.Linear, DeviceContext) classes.
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   constexpr Py_ssize_t kFns = sizeof(Abi) / sizeof(void*);
+  PyTypeObject** types[] = {&t_router, &t_experts, &t_mlp, &t_block, &t_linear, &t_device_context};
+  constexpr Py_ssize_t kTypes = sizeof(types) / sizeof(*types);
   if (n != 2 || !PyTuple_CheckExact(args[0]) || PyTuple_GET_SIZE(args[0]) != kFns ||
-      !PyTuple_CheckExact(args[1]) || PyTuple_GET_SIZE(args[1]) != 5) {
+      !PyTuple_CheckExact(args[1]) || PyTuple_GET_SIZE(args[1]) != kTypes) {
     PyErr_SetString(PyExc_TypeError, "bind(entry point addresses, module classes)");
     return nullptr;
   }
@@ -455,13 +470,12 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
       return nullptr;
     }
   }
-  PyTypeObject** types[5] = {&t_router, &t_experts, &t_mlp, &t_block, &t_linear};
-  for (int i = 0; i < 5; ++i)
+  for (Py_ssize_t i = 0; i < kTypes; ++i)
     if (!PyType_Check(PyTuple_GET_ITEM(args[1], i))) {
       PyErr_SetString(PyExc_TypeError, "bind: classes expected");
       return nullptr;
     }
-  for (int i = 0; i < 5; ++i) {
+  for (Py_ssize_t i = 0; i < kTypes; ++i) {
     PyObject* old = reinterpret_cast<PyObject*>(*types[i]);
     *types[i] = reinterpret_cast<PyTypeObject*>(Py_NewRef(PyTuple_GET_ITEM(args[1], i)));
     Py_XDECREF(old);
@@ -477,6 +491,7 @@ PyMethodDef methods[] = {
     {"router", reinterpret_cast<PyCFunction>(router), METH_FASTCALL, nullptr},
     {"experts", reinterpret_cast<PyCFunction>(experts), METH_FASTCALL, nullptr},
     {"mlp", reinterpret_cast<PyCFunction>(mlp), METH_FASTCALL, nullptr},
+    {"plain", plain, METH_NOARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods,

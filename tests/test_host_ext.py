@@ -34,6 +34,24 @@ def test_left_to_the_general_path_on_cpu(lbmoe):
     assert h.mlp(b.shared_expert) is None                 # a wrong argument count
 
 
+def test_a_default_device_is_no_mode_to_decline(lbmoe):
+    """torch.set_default_device leaves a DeviceContext on the mode stack for good: it changes no call
+    that names its devices, so it must not send every call to the general path."""
+    h = moe._host()
+    assert h.plain()
+    with torch.device("cpu"):
+        assert h.plain()
+        with _Mode():
+            assert not h.plain()
+    torch.set_default_device("cpu")
+    try:
+        assert torch._C._len_torch_function_stack() == 1 and h.plain()
+    finally:
+        torch.set_default_device(None)
+    with _Mode(), torch.device("meta"):
+        assert not h.plain()
+
+
 class _Norm(torch.nn.Module):
     eps = 1e-6
 
@@ -78,6 +96,24 @@ def test_same_results_as_the_general_path(gpu, monkeypatch, Is, fp8, bias, T):
     monkeypatch.setattr(moe, "_host", lambda: _Declines())
     for a, c in zip(fast, _calls(*args)):
         assert a.dtype == c.dtype and torch.equal(a, c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("default", ["cpu", "cuda"])
+def test_taken_under_a_default_device(gpu, default):
+    b, h, norm = _block(gpu), moe._host(), _Norm(gpu)
+    g = torch.Generator().manual_seed(3)
+    x, res = make_x(g, 3, 512).to(gpu), make_x(g, 3, 512).to(gpu)
+    tw, idx = b.gate(x)
+    want = _calls(b, x, res, norm, idx, tw)
+    torch.set_default_device(default)
+    try:
+        got = [h.block(b, x, None), *h.block_norm(b, x, res, norm, None), *h.router(b.gate, x),
+               h.experts(b.experts, x, idx, tw), h.mlp(b.shared_expert, x)]
+    finally:
+        torch.set_default_device(None)
+    for a, c in zip(got, want, strict=True):
+        assert a.device == gpu and torch.equal(a, c)
 
 
 @pytest.mark.gpu
