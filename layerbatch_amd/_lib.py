@@ -3,10 +3,13 @@
 torch is imported first so that the library's libamdhip64 dependency resolves to the HIP
 runtime torch already loaded (same SONAME): device pointers and streams from torch are then
 valid in the library. The library must have been built in-tree
-(``python -m layerbatch_amd.build``); there is no fallback implementation.
+(``python -m layerbatch_amd.build``); there is no fallback implementation. The host extension
+built with it only shortens the module calls' host side: without it they take moe.py's general
+path to the same library.
 """
 import ctypes
 import os
+import warnings
 
 import torch  # noqa: F401  (must precede the library load, see module docstring)
 
@@ -93,21 +96,41 @@ def lib():
     return _lib
 
 
+class _NoHost:
+    """Stands in for a host extension that does not load: it takes no call."""
+
+    @staticmethod
+    def block(*args):
+        return None
+
+    block_norm = router = experts = mlp = block
+
+
 def host(classes):
     """The host extension (csrc/host_ext.cpp), bound to the library and to the module classes
-    (router, experts, shared-expert MLP, block)."""
+    (router, experts, shared-expert MLP, block). Where it is missing or was built against another
+    torch, a stand-in that leaves every call to the general path, with one warning: that path is
+    complete, its calls cost the host some 40 us more."""
     global _host
     if _host is None:
         h = lib()
         try:
             from torch.utils._device import DeviceContext
             from . import _host as ext
+            mine = ".".join(torch.__version__.split("+")[0].split(".")[:2])
+            why = None if ext.torch_version == mine else (
+                f"it was built against torch {ext.torch_version}, this is {mine}")
         except ImportError as e:
-            raise RuntimeError(f"the host extension does not load ({e}): build it with "
-                               "`python -m layerbatch_amd.build`") from e
-        ext.bind(tuple(ctypes.cast(getattr(h, n), _p).value for n in _HOST_FNS),
-                 (*classes, torch.nn.Linear, DeviceContext))
-        _host = ext
+            why = str(e)
+        if why is None:
+            ext.bind(tuple(ctypes.cast(getattr(h, n), _p).value for n in _HOST_FNS),
+                     (*classes, torch.nn.Linear, DeviceContext))
+            _host = ext
+        else:
+            warnings.warn(f"the host extension does not load ({why}): module calls take the slower "
+                          "Python path; build it with `python -m layerbatch_amd.build`",
+                          RuntimeWarning, stacklevel=2)
+            _host = _NoHost()
     return _host
 
 

@@ -12,6 +12,7 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import warnings
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
@@ -48,12 +49,30 @@ def _compile(hipcc, src):
     return obj, warn
 
 
-def _build_host():
-    """Compile and link the host extension against the installed torch."""
+def _host_cxx(hipcc):
+    """A host C++ compiler: CXX, the system's, or the clang++ that hipcc itself runs; or None."""
+    near = os.path.dirname(os.path.realpath(hipcc))
+    for cand in (os.environ.get("CXX"), "g++", "c++", os.path.join(near, "amdclang++"),
+                 os.path.join(near, "..", "llvm", "bin", "clang++"), "clang++"):
+        path = shutil.which(cand) if cand else None
+        if path:
+            return path
+    return None
+
+
+def _build_host(hipcc):
+    """Compile and link the host extension against the installed torch. Without a host compiler or
+    Python's headers none is left in place: the module calls then take the general Python path."""
     import torch
-    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
-    if not cxx:
-        raise RuntimeError("no host C++ compiler found (set CXX)")
+    cxx = _host_cxx(hipcc)
+    python_h = os.path.join(sysconfig.get_paths()["include"], "Python.h")
+    if not cxx or not os.path.exists(python_h):
+        warnings.warn("the host extension is not built: "
+                      + ("no host C++ compiler found (set CXX)" if not cxx else f"no {python_h}"),
+                      RuntimeWarning, stacklevel=2)
+        if os.path.exists(HOST):
+            os.remove(HOST)
+        return
     root = os.path.dirname(torch.__file__)
     inc, rocm = os.path.join(root, "include"), os.environ.get("ROCM_PATH", "/opt/rocm")
     tmp = HOST + ".tmp"
@@ -76,7 +95,7 @@ def build(verbose=False):
     os.makedirs(BUILD, exist_ok=True)
     srcs = sources()
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
-        host = ex.submit(_build_host)
+        host = ex.submit(_build_host, hipcc)
         results = list(ex.map(lambda s: _compile(hipcc, s), srcs))
         host.result()
     for obj, warn in results:

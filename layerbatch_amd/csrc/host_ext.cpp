@@ -25,6 +25,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/utils/pybind.h>
+#include <torch/headeronly/version.h>
 
 #include <cstring>
 #include <optional>
@@ -499,6 +500,9 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods,
 
 }  // namespace
 
+#define LBMOE_STR1(x) #x
+#define LBMOE_STR(x) LBMOE_STR1(x)
+
 PyMODINIT_FUNC PyInit__host(void) {
   PyObject** names[] = {&nm.parameters, &nm.modules, &nm.weight, &nm.bias, &nm.gate, &nm.experts,
                         &nm.shared_expert, &nm.shared_expert_gate, &nm.gate_proj, &nm.up_proj,
@@ -517,5 +521,10 @@ PyMODINIT_FUNC PyInit__host(void) {
     *names[i] = PyUnicode_InternFromString(text[i]);
     if (!*names[i]) return nullptr;
   }
-  return PyModule_Create(&module_def);
+  PyObject* m = PyModule_Create(&module_def);
+  // the torch whose headers this was compiled with: _lib.py loads no other
+  constexpr const char* kTorch =
+      LBMOE_STR(TORCH_VERSION_MAJOR) "." LBMOE_STR(TORCH_VERSION_MINOR);
+  if (m && PyModule_AddStringConstant(m, "torch_version", kTorch) < 0) Py_CLEAR(m);
+  return m;
 }

@@ -14,10 +14,10 @@ def pytest_configure(config):
 
 @pytest.fixture(scope="session")
 def lbmoe():
-    """The loaded C-ABI library; built in-tree first when hipcc is present and it is missing."""
-    from layerbatch_amd import _lib
-    if not os.path.exists(_lib.LIB_PATH):
-        from layerbatch_amd import build
+    """The loaded C-ABI library; built in-tree first when hipcc is present and it or the host
+    extension is missing."""
+    from layerbatch_amd import _lib, build
+    if not (os.path.exists(_lib.LIB_PATH) and os.path.exists(build.HOST)):
         build.build()
     return _lib.lib()
 

@@ -1,9 +1,14 @@
 """The host extension against the general Python path: the plain calls it takes give the same bits,
 and everything else is left to the general path (None), on the CPU and under torch's modes."""
+import os
+import sys
+import types
+
 import pytest
 import torch
 
-from layerbatch_amd import moe
+import layerbatch_amd
+from layerbatch_amd import _lib, build, moe
 from layerbatch_amd.synth import MoEShape, make_layer, make_x
 
 
@@ -50,6 +55,49 @@ def test_a_default_device_is_no_mode_to_decline(lbmoe):
         torch.set_default_device(None)
     with _Mode(), torch.device("meta"):
         assert not h.plain()
+
+
+@pytest.mark.parametrize("ext,why", [
+    (None, "_host"), (types.SimpleNamespace(torch_version="1.0"), "built against torch 1.0")])
+def test_the_general_path_runs_without_the_extension(lbmoe, monkeypatch, ext, why):
+    """An extension that is missing, or was built against another torch, is left out with one
+    warning; the calls (refused ones here, on the CPU) reach the general path."""
+    monkeypatch.setattr(_lib, "_host", None)
+    if ext is None:
+        monkeypatch.delattr(layerbatch_amd, "_host", raising=False)
+        monkeypatch.setitem(sys.modules, "layerbatch_amd._host", None)
+    else:
+        monkeypatch.setattr(layerbatch_amd, "_host", ext, raising=False)
+        monkeypatch.setitem(sys.modules, "layerbatch_amd._host", ext)
+    b, x = _block("cpu"), torch.zeros((3, 512), dtype=torch.bfloat16)
+    with pytest.warns(RuntimeWarning, match=why) as caught:
+        for call in (b, b.gate, b.shared_expert, lambda v: b.forward_norm(v, v, None),
+                     lambda v: b.experts(v, None, None)):
+            with pytest.raises(RuntimeError, match="is on cpu"):
+                call(x)
+    assert len(caught) == 1
+    assert _lib.host(()).block(b, x, None) is None
+
+
+def test_build_without_a_host_compiler(monkeypatch, tmp_path):
+    """Any C++ compiler will do, hipcc's own too; with none the library is still built and no stale
+    extension stays behind."""
+    stale = tmp_path / "_host.so"
+    stale.write_bytes(b"")
+    monkeypatch.setattr(build, "HOST", str(stale))
+    monkeypatch.delenv("CXX", raising=False)
+    rocm = tmp_path / "bin"
+    rocm.mkdir()
+    hipcc = rocm / "hipcc"
+    monkeypatch.setenv("PATH", str(tmp_path / "empty"))
+    assert build._host_cxx(str(hipcc)) is None
+    with pytest.warns(RuntimeWarning, match="no host C\\+\\+ compiler"):
+        build._build_host(str(hipcc))
+    assert not stale.exists()
+    clang = rocm / "amdclang++"
+    clang.write_text("#!/bin/sh\n")
+    os.chmod(clang, 0o755)
+    assert build._host_cxx(str(hipcc)) == str(clang)
 
 
 class _Norm(torch.nn.Module):
