@@ -13,7 +13,8 @@
  *    point only enqueues work on that stream: no host synchronisation, no device
  *    allocation, grids that depend on T and the layer shape only. The entry points are
  *    therefore safe inside HIP graph capture and on any caller-chosen stream.
- *  - Scratch memory is caller-owned: size it with lbmoe_workspace_size and pass it in.
+ *  - Scratch memory is caller-owned: size it with lbmoe_workspace_size and pass it in, on a
+ *    4-byte boundary at least (it holds int32 arrays; every allocator gives more).
  *  - Every entry point returns an lbmoe_status; a negative value means nothing was
  *    enqueued (argument errors) or the launch failed. There is no fallback path.
  *  - The library's only global state is set once per device and then read: the
@@ -38,7 +39,8 @@ typedef enum lbmoe_status {
   LBMOE_ERR_NULL = -1,        /* a required pointer is NULL                         */
   LBMOE_ERR_SHAPE = -2,       /* unsupported or inconsistent sizes                  */
   LBMOE_ERR_DTYPE = -3,       /* unknown weight dtype / index width                 */
-  LBMOE_ERR_WORKSPACE = -4,   /* workspace smaller than lbmoe_workspace_size        */
+  LBMOE_ERR_WORKSPACE = -4,   /* workspace smaller than lbmoe_workspace_size, or (of a
+                                 layer call) not on a 4-byte boundary               */
   LBMOE_ERR_DEVICE = -5,      /* current device is not gfx950 / no device           */
   LBMOE_ERR_LAUNCH = -6,      /* a kernel launch reported an error                  */
   LBMOE_ERR_STATIC_LIMIT = -7 /* lbmoe_forward_static: the call needs more workspace than

@@ -117,6 +117,13 @@ static int32_t check_shared_ptrs(const lbmoe_layer& L) {
   return LBMOE_OK;
 }
 
+// The int32 regions of a workspace that starts between 4-byte boundaries would be misread: row counts,
+// offsets and dispatch entries come through scalar loads, which drop an address's two low bits, and a
+// wrong count sends the GEMMs out of range.
+static int32_t check_workspace(const void* ws, size_t bytes, size_t need) {
+  return bytes < need || (reinterpret_cast<uintptr_t>(ws) & 3) != 0 ? LBMOE_ERR_WORKSPACE : LBMOE_OK;
+}
+
 static int32_t check_T(const lbmoe_layer& L, int64_t T) {
   if (T < 0 || T > (int64_t{1} << 21)) return LBMOE_ERR_SHAPE;
   if (T * (L.top_k + 1) > INT32_MAX) return LBMOE_ERR_SHAPE;
@@ -345,7 +352,7 @@ const char* lbmoe_status_string(int32_t status) {
     case LBMOE_ERR_NULL: return "required pointer is NULL";
     case LBMOE_ERR_SHAPE: return "unsupported or inconsistent shape";
     case LBMOE_ERR_DTYPE: return "unsupported dtype or index width";
-    case LBMOE_ERR_WORKSPACE: return "workspace too small";
+    case LBMOE_ERR_WORKSPACE: return "workspace too small or not on a 4-byte boundary";
     case LBMOE_ERR_DEVICE: return "current device is not gfx950";
     case LBMOE_ERR_LAUNCH: return "kernel launch failed";
     case LBMOE_ERR_STATIC_LIMIT:
@@ -454,7 +461,7 @@ static int32_t forward_impl(const lbmoe_layer* layer, const void* x, int64_t T, 
   if (T == 0) return LBMOE_OK;
   if (!x || !y || !workspace) return LBMOE_ERR_NULL;
   const WsLayout w = ws_layout(L, T);
-  if (workspace_bytes < w.total) return LBMOE_ERR_WORKSPACE;
+  if ((st = check_workspace(workspace, workspace_bytes, w.total)) != LBMOE_OK) return st;
   if ((st = check_device()) != LBMOE_OK) return st;
   hipStream_t s = static_cast<hipStream_t>(stream);
   void* ws = workspace;
@@ -650,7 +657,7 @@ int32_t lbmoe_experts(const lbmoe_layer* layer, const void* x, const void* topk_
   if (T == 0) return LBMOE_OK;
   if (!x || !topk_idx || !topk_w || !y || !workspace) return LBMOE_ERR_NULL;
   const WsLayout w = ws_layout(L, T);
-  if (workspace_bytes < w.total) return LBMOE_ERR_WORKSPACE;
+  if ((st = check_workspace(workspace, workspace_bytes, w.total)) != LBMOE_OK) return st;
   if ((st = check_device()) != LBMOE_OK) return st;
   return run_experts(L, x, topk_idx, idx_bytes, topk_w, nullptr, T, y, workspace, w, false,
                      static_cast<hipStream_t>(stream));

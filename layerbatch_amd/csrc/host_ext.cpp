@@ -307,7 +307,9 @@ PyObject* run_block(PyObject* mod, PyObject* px, PyObject* pres, PyObject* pnorm
   at::Tensor ws;
   if (pws != Py_None) {
     const at::Tensor* w = ts.add(pws);
-    if (!w || w->scalar_type() != at::kByte || !w->is_contiguous()) Py_RETURN_NONE;
+    if (!w || w->scalar_type() != at::kByte || !w->is_contiguous() ||
+        (reinterpret_cast<uintptr_t>(w->const_data_ptr()) & 3) != 0)
+      Py_RETURN_NONE;
     ws = *w;
   }
   at::Tensor y, res_out;

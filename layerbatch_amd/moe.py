@@ -104,12 +104,15 @@ def _same_device(module, device):
 
 def _workspace(layer, T, device, workspace=None):
     """The caller's workspace (checked: uint8, contiguous, on the input's device; the library
-    checks its size), or a new one from torch's caching allocator."""
+    checks its size), or a new one from torch's caching allocator, also in the place of a view
+    that starts between 4-byte boundaries, where the library's int32 arrays cannot lie."""
     if workspace is None:
         return torch.empty(_lib.workspace_size(layer, T), dtype=torch.uint8, device=device)
     _require(workspace, "workspace", torch.uint8)
     if workspace.device != device:
         raise RuntimeError(f"workspace is on {workspace.device}, the input on {device}")
+    if workspace.data_ptr() % 4 and workspace.numel() >= _lib.workspace_size(layer, T):
+        return _workspace(layer, T, device)
     return workspace
 
 

@@ -175,6 +175,29 @@ def test_forward_rejects_bad_arguments_before_any_device_call(lbmoe):
     assert lbmoe.lbmoe_dense_mlp(p, p, p, None, None, None, 1024, 0, 0, p, 4, p, p, 1 << 20, None) == ERR_SHAPE
 
 
+def test_workspace_between_4_byte_boundaries_is_refused(lbmoe):
+    """Its int32 regions come through scalar loads, which drop an address's low bits."""
+    import torch
+    from layerbatch_amd import moe
+    L, n, p = _layer(), ctypes.c_size_t(0), ctypes.c_void_p(0x10000)
+    lbmoe.lbmoe_workspace_size(ctypes.byref(L), 16, ctypes.byref(n))
+    for off in (1, 2, 3):
+        ws = ctypes.c_void_p(0x10000 + off)
+        assert lbmoe.lbmoe_forward(ctypes.byref(L), p, 16, p, ws, n.value, None) == ERR_WORKSPACE
+        assert lbmoe.lbmoe_forward_norm(ctypes.byref(L), p, ctypes.c_void_p(0x20000), p, 1e-6, 16, p,
+                                        ctypes.c_void_p(0x30000), ws, n.value, None) == ERR_WORKSPACE
+        assert lbmoe.lbmoe_experts(ctypes.byref(L), p, p, 4, p, 16, p, ws, n.value, None) == ERR_WORKSPACE
+    # the modules put a new one in the place of such a view, and leave one too small to be refused
+    base = torch.zeros(n.value + 8, dtype=torch.uint8)
+    view = base[1 + -base.data_ptr() % 4:][:n.value]
+    assert view.data_ptr() % 4 == 1
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(moe, "_require", lambda *a: None)
+        assert moe._workspace(L, 16, base.device, view).data_ptr() % 4 == 0
+        assert moe._workspace(L, 16, base.device, view[:-1]).data_ptr() == view.data_ptr()
+        assert moe._workspace(L, 16, base.device, base) is base
+
+
 def test_pack_weights_rejects_bad_arguments_before_any_device_call(lbmoe):
     p = ctypes.c_void_p(0x10000)
     L = _layer()
