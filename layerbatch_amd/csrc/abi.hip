@@ -305,8 +305,7 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
     LBMOE_TRY(ev->mark(s));
     return LBMOE_OK;
   }
-  if (rt && use_tiled(L, gw, x, T, k)) return LBMOE_ERR_SHAPE;   // not reached (see forward_impl)
-  if (use_tiled(L, gw, x, T, k)) {
+  if (!rt && use_tiled(L, gw, x, T, k)) {
     // prefill-sized batch: LDS-tiled MFMA GEMMs over a device-built token-tile list
     if (!tiles_built)
       LBMOE_TRY(launch_build_tiles(counts, offsets, gw, with_shared, T, max_tiles, tiles, s));

@@ -17,7 +17,6 @@ struct PermSingleLds {
   alignas(16) int cnt[kVW][EMAX];                     // per virtual wave and expert: count, prefix
   int psum[kParts][EMAX];
   int start[EMAX];                                    // first row of each expert
-  int total[EMAX];                                    // rows of each expert
   int wsum[kW];
 };
 
@@ -115,7 +114,6 @@ __device__ __forceinline__ void perm_single_body(PermSingleLds<R, EMAX>& lds, co
   const int excl = before + incl - total;
   if (tid < E) {
     lds.start[tid] = excl;
-    lds.total[tid] = total;
     counts[tid] = total;
     offsets[tid] = excl;
   }

@@ -9,8 +9,8 @@
 // r; OCP e4m3 operands, unit E8M0 scales). Its product p is scaled by
 // w_scale(row block, k-tile) * a_scale(token, k-tile) and added to the fp32 accumulator; the
 // fused multiply-adds of one MFMA step run under the next step's MFMAs.
-// Workgroup: 8 waves in 2 x 4, kWM = 256 weight rows x 256 tokens (wide: a wave owns 128 rows
-// x 64 tokens, 8 x 4 tiles of 16 x 16), x 128 tokens (narrow: 128 x 32) or, on 4 x 2 waves,
+// Workgroup: 8 waves and kWM = 256 weight rows, x 256 tokens on 2 x 4 waves (wide: a wave owns 128
+// rows x 64 tokens, 8 x 4 tiles of 16 x 16) or, on 4 x 2 waves, x 128 tokens (narrow: 64 x 64) or
 // x 64 tokens (tiny: 64 x 32). Accumulator lane (r, q) of a tile holds token column r and
 // rows 4q .. 4q+3.
 // Scales live in LDS for the whole work item: the activation scales of the tile's tokens for

@@ -182,8 +182,8 @@ __device__ __forceinline__ void write_dispatch(const int* list, const int2* grp,
 // Tile lists up to this many entries are also assembled in LDS, where the dispatch tables
 // read them back; longer ones are read back from memory. With the list in LDS, up to
 // kBuildBlocks workgroups write the dispatch tables: each assembles the (short) list itself and
-// writes its share of the entries, so the table loop (two 64-bit divisions per entry) does not
-// hold one CU for the whole launch. Workgroup 0 alone writes the list, its counts and the queues.
+// writes its share of the entries, so the table loop (two divisions per entry, in dispatch_item)
+// does not hold one CU for the whole launch. Workgroup 0 alone writes the list, its counts and the queues.
 constexpr int kLdsListEntries = 4096;
 constexpr int kBuildBlocks = 32;
 constexpr int kBuildEntriesPerBlock = 256;
@@ -549,8 +549,8 @@ __device__ __forceinline__ void store_partial(const f32x16 (&acc)[S::kMT][S::kNT
 // PARTIAL (router only): only k-tiles kt0 .. kt0 + nkt - 1 of the product, whose fp32 sums go
 // to part (store_partial) instead of logits.
 // KS > 1 (small dense and router tiles): the workgroup has KS groups of S::kNumWaves waves, each
-// with its own ring over 1 / KS of the k range; the groups' fp32 sums meet in LDS (group_sums) and
-// are added in group order, each group finishing its share of the tile.
+// with its own ring over 1 / KS of the k range; the groups' fp32 sums meet in LDS and are added in
+// group order, each group finishing its share of the tile.
 // DENSE: the dense MLP (dense_tiled_kernel): one group whose weights every token tile reads and
 // whose output rows the caller reads next, so neither takes the non-temporal policies.
 template <int MODE, class S, int kLdsCap = kLdsU4, bool PERSIST = false, bool STAGE = false,
