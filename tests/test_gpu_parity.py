@@ -447,14 +447,30 @@ class _Norm(torch.nn.Module):
                                           ("qwen3-30b-a3b", 1), ("qwen3-30b-a3b", 16),
                                           ("small-h1024-e16", 13), ("qwen3-next-e512", 1100)])
 def test_forward_norm(gpu, shape_name, T):
+    _check_forward_norm(gpu, SHAPES[shape_name], T)
+
+
+# T >= 1024 with at most 128 experts on the tiled GEMMs: the norm's own kernel, then the router that
+# also selects (k range split over workgroups, or from 16384 tokens whole), which reads the normalised
+# rows for the logits and for the shared expert's gate
+@pytest.mark.parametrize("shape,T,fp8", [
+    (SHAPES["small-h1024-e16"], 1100, False), (SHAPES["qwen3-30b-a3b"], 1024, False),
+    (MoEShape(512, 64, 4, 256, 256), 1501, False), (MoEShape(512, 32, 2, 256, 256), 1300, True),
+    (MoEShape(512, 20, 2, 256, 128), 16391, False)])
+def test_forward_norm_fused_router(gpu, shape, T, fp8):
+    _check_forward_norm(gpu, shape, T, fp8)
+
+
+def _check_forward_norm(gpu, shape, T, fp8=False):
     """Residual add + RMSNorm + block (qwen3_5.py:998-1004): the new residual is the bf16 sum
     bit for bit, the block input within one bf16 step of the oracle's Qwen3_5RMSNorm, and the
     output equals the plain block on that input bit for bit (decode T: norm fused into the
-    router kernel; T >= 1024: separate norm kernel)."""
-    shape = SHAPES[shape_name]
+    router kernel; more tokens: separate norm kernel)."""
     H = shape.hidden_size
     w, g = make_layer(shape, seed=T, device=gpu)
     blk = _block(shape, w, gpu)
+    if fp8:
+        blk.quantize_fp8_()
     hid = make_x(g, T, H, device=gpu)
     res = (make_x(g, T, H, device=gpu).float() * 3).to(torch.bfloat16)
     norm = _Norm((make_x(g, 1, H, device=gpu)[0].float() * 0.1).to(torch.bfloat16), 1e-6)
