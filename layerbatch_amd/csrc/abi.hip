@@ -5,10 +5,10 @@
 
 #include <algorithm>
 #include <atomic>
-#include <cmath>
 #include <cstring>
 
 #include "internal.hpp"
+#include "rules.hpp"
 
 namespace lbmoe {
 
@@ -166,40 +166,15 @@ static P* at(void* ws, const WsLayout& w, int r) {
     if ((expr) != hipSuccess) return LBMOE_ERR_LAUNCH;        \
   } while (0)
 
-// Expected tokens per routed expert from which the LDS-tiled GEMMs replace weight streaming. The
-// streaming kernels run two token tiles per pass above 8 tokens per expert and four above 28, each
-// step slower; the tiled ones barely depend on the count, but their items (one per expert and 128
-// intermediate channels at these sizes) must fill whole rounds of the CUs. Measured (GPU us per layer
-// call, streaming / tiled):
-//   bf16, 8 items per CU (E = 512, I = 512): 7.5 tokens per expert 535 / 531, 20 tokens 639 / 565
-//   bf16, 3 and 2, whole rounds (E = 128, I = 768; E = 256, I = 256): 10 tokens 204 / 207 and 104 /
-//     106, 14 tokens 218 / 209 and 111 / 109
-//   bf16, 2.25 and 1.5 (the last round three quarters full or less): 12 tokens 173 / 183 and 113 / 117,
-//     20 tokens 197 / 186 and 126 / 120; 0.75: 17 tokens 80 / 79
-//   bf16, 1.17 and 1.25: 15 tokens 103 / 118 and 70 / 73, 27 tokens 137 / 123
-//   fp8 (its streaming kernels stream less per wave): 10 tokens 339 / 328 (8 items per CU) and 82 /
-//     81 (2), 12 tokens 149 / 129 (3) and 61 / 50 (0.75)
-// Below 0.7 items per CU the tiled launches leave CUs idle and only the four-tile passes are slower
-// (E = 16, I = 512: 25 tokens 32 / 36). Skewed routings gain more: under a Zipf bias the streaming
-// kernels walk a popular expert's rows pass after pass (E = 512, 7.5 tokens: 477 / 139).
+// Whether the call's experts run on the LDS-tiled GEMMs (tiled_min_tokens).
 // Below kTiledAlways only operands on 16-byte boundaries (of the copies) leave the streaming kernels.
-constexpr double kTiledAlways = 28.0;
-static double tiled_min_tokens(const GroupWeights& gw, bool fp8) {
-  const double n = static_cast<double>(gw.E) * (gw.I / 128) / device_cus();   // items per CU
-  const double full = n / std::ceil(n);
-  if (fp8) return n >= 0.7 ? 10.0 : kTiledAlways;
-  if (n >= 4.0) return 8.0;
-  if (full >= 0.9 && n >= 1.0) return 13.0;
-  if (full >= 0.7) return 17.0;
-  return n >= 1.0 ? 24.0 : kTiledAlways;
-}
-
 static bool use_tiled(const lbmoe_layer& L, const GroupWeights& gw, const void* x, int64_t T,
                       int k) {
   if (!tiled_supported(gw) || !tiled_offsets_fit(gw, T, k)) return false;
   const double avg = static_cast<double>(T) * k / gw.E;
   if (avg >= kTiledAlways) return true;
-  return avg >= tiled_min_tokens(gw, is_fp8(L)) &&
+  const CallSizes c{gw.E, gw.H, gw.I, gw.groups > gw.E ? gw.Is : 0, T, is_fp8(L), device_cus()};
+  return avg >= tiled_min_tokens(c) &&
          aligned16({x, gw.gate_up, gw.down, gw.sh_gate, gw.sh_up, gw.sh_down});
 }
 

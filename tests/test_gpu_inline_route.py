@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
     (MoEShape(1024, 16, 2, 256, 0), 8),        # both apply: routed in gate_up
     (MoEShape(1024, 32, 3, 256, 0), 10),       # T * k < E
     (MoEShape(1024, 32, 2, 256, 128), 16),     # T * k = E
-    (MoEShape(256, 2, 2, 65536, 0), 8),        # 8 tokens per expert on the tiled GEMMs: not routed inside
+    (MoEShape(256, 2, 2, 65536, 0), 8),        # the largest width
+    (MoEShape(256, 2, 2, 32768, 65536), 8),    # 8 tokens per expert on the tiled GEMMs: not routed inside
 ])
 def test_small_batches(gpu, shape, T):
     _run_and_check(shape, T, gpu, seed=T + shape.num_experts)

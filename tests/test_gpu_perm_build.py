@@ -11,6 +11,7 @@ from layerbatch_amd.synth import MoEShape, make_layer, make_x
 from oracle import moe as om
 from tests import gpu_checks as gc
 from tests.helpers import layer_np, to_np
+from tests.test_gpu_fp8 import _run_fp8
 from tests.test_gpu_parity import _block, _run_and_check
 
 pytestmark = pytest.mark.gpu
@@ -65,13 +66,26 @@ def test_experts_perm_build(gpu, T, k, E, dt):
     gc.check_output(to_np(y)[rows], ref, gc.TOL_BF16)
 
 
-# tokens per expert on either side of the switch: 8 items per CU, whole rounds, partly filled ones
+# (shape, T, fp8): T is the first batch on the LDS-tiled GEMMs (test_dispatch_rules checks that): whole
+# and partly filled rounds of the CUs, less than one, the shared expert's items past a whole round
+SWITCH = [(MoEShape(256, 512, 2, 512, 128), 2509, False), (MoEShape(256, 256, 4, 256, 0), 512, False),
+          (MoEShape(256, 96, 2, 512, 128), 767, False), (MoEShape(1024, 128, 4, 512, 512), 587, False),
+          (MoEShape(256, 128, 4, 256, 0), 352, True), (MoEShape(512, 64, 4, 512, 256), 413, True),
+          (MoEShape(1024, 48, 4, 768, 0), 120, True), (MoEShape(768, 100, 3, 512, 256), 372, True)]
+
+
 @pytest.mark.parametrize("shape,T", [
     (MoEShape(256, 512, 2, 512, 128), 2047), (MoEShape(256, 512, 2, 512, 128), 2048),
     (MoEShape(256, 256, 4, 256, 0), 831), (MoEShape(256, 256, 4, 256, 0), 832),
-    (MoEShape(256, 96, 2, 512, 128), 815), (MoEShape(256, 96, 2, 512, 128), 816)])
+    (MoEShape(256, 96, 2, 512, 128), 815), (MoEShape(256, 96, 2, 512, 128), 816)]
+    + [(s, t - d) for s, t, fp8 in SWITCH if not fp8 for d in (1, 0)])
 def test_block_at_the_switch(gpu, shape, T):
     _run_and_check(shape, T, gpu, seed=T, sample=48)
+
+
+@pytest.mark.parametrize("shape,T", [(s, t - d) for s, t, fp8 in SWITCH if fp8 for d in (1, 0)])
+def test_fp8_block_at_the_switch(gpu, shape, T):
+    _run_fp8(shape, T, gpu, seed=T, sample=48)
 
 
 def test_unaligned_rows_at_the_switch(gpu):
