@@ -166,16 +166,23 @@ static P* at(void* ws, const WsLayout& w, int r) {
     if ((expr) != hipSuccess) return LBMOE_ERR_LAUNCH;        \
   } while (0)
 
-// Whether the call's experts run on the LDS-tiled GEMMs (tiled_min_tokens).
-// Below kTiledAlways only operands on 16-byte boundaries (of the copies) leave the streaming kernels.
-static bool use_tiled(const lbmoe_layer& L, const GroupWeights& gw, const void* x, int64_t T,
-                      int k) {
+// Whether the call's experts run on the LDS-tiled GEMMs (tiled_min_tokens). Their copies take operands
+// at any address, but weights between 16-byte boundaries cost them more than the streaming kernels, so
+// those leave the latter from kTiledAlways only (Qwen3-30B-A3B, us streaming / tiled: T = 256 weights 8
+// bytes off 295 / 345, packed copies 2 bytes off 230 / 279; T = 1000 561 / 382. Token rows 2 bytes off
+// 270 / 217, workspace 4 bytes off 236 / 215).
+static bool use_tiled(const lbmoe_layer& L, const GroupWeights& gw, int64_t T, int k) {
   if (!tiled_supported(gw) || !tiled_offsets_fit(gw, T, k)) return false;
   const double avg = static_cast<double>(T) * k / gw.E;
   if (avg >= kTiledAlways) return true;
-  const CallSizes c{gw.E, gw.H, gw.I, gw.groups > gw.E ? gw.Is : 0, T, is_fp8(L), device_cus()};
-  return avg >= tiled_min_tokens(c) &&
-         aligned16({x, gw.gate_up, gw.down, gw.sh_gate, gw.sh_up, gw.sh_down});
+  const bool sh = gw.groups > gw.E;
+  const CallSizes c{gw.E, gw.H, gw.I, sh ? gw.Is : 0, T, is_fp8(L), device_cus()};
+  if (avg < tiled_min_tokens(c)) return false;
+  auto copied = [](const void* packed, const void* w) { return packed ? packed : w; };
+  return aligned16({copied(gw.gate_up_tiled, gw.gate_up), copied(gw.down_tiled, gw.down)}) &&
+         (!sh || aligned16({copied(gw.sh_gate_up_tiled, gw.sh_gate),
+                            copied(gw.sh_gate_up_tiled, gw.sh_up),
+                            copied(gw.sh_down_tiled, gw.sh_down)}));
 }
 
 // Routed experts of one call: permute, gate_up, down, combine.
@@ -214,7 +221,7 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
   if (T * k < E) gw.hit_rows = static_cast<int>(T * k);
   // the route's own ids (all in [0, E)) can be permuted inside the bf16 decode gate_up kernel
   const bool perm_in_gate_up = own_ids && !permuted && idx_bytes == 4 && !is_fp8(L) &&
-                               !use_tiled(L, gw, x, T, k) && gate_up_perm_supported(gw, T, k);
+                               !use_tiled(L, gw, T, k) && gate_up_perm_supported(gw, T, k);
   int32_t* tiles = at<int32_t>(ws, w, R_TILES);
   const int max_tiles = tiled_max_tiles(T * k + (with_shared ? T : 0), gw.groups);
   bool tiles_built = false;
@@ -228,7 +235,7 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
                                    max_tiles, tiles, s));
     tiles_built = true;
   } else if (!permuted && !perm_in_gate_up) {
-    const bool tiled = use_tiled(L, gw, x, T, k) &&
+    const bool tiled = use_tiled(L, gw, T, k) &&
                        (!is_fp8(L) || tiled_fp8_supported(gw, T, T * k + (with_shared ? T : 0)));
     if (tiled && perm_build_supported(T * k, T, max_tiles)) {
       LBMOE_TRY(launch_perm_build(idx, idx_bytes, T, k, counts, offsets, perm_tok,
@@ -262,7 +269,7 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
     float* acts = at<float>(ws, w, R_ACTS);
     const int64_t rows = T * k + (with_shared ? T : 0);
     if (!x_quantised) LBMOE_TRY(launch_quant_groups_fp8(x, T, H, H, xq, xs, s));
-    if (use_tiled(L, gw, x, T, k) && tiled_fp8_supported(gw, T, rows)) {
+    if (use_tiled(L, gw, T, k) && tiled_fp8_supported(gw, T, rows)) {
       if (!tiles_built)
         LBMOE_TRY(launch_build_tiles(counts, offsets, gw, with_shared, T, max_tiles, tiles, s));
       LBMOE_TRY(launch_gate_up_tiled_fp8(gw, xq, xs, perm_tok, tiles, max_tiles, Imax, actq, acts,
@@ -280,7 +287,7 @@ static int32_t run_experts(const lbmoe_layer& L, const void* x, const void* idx,
     LBMOE_TRY(ev->mark(s));
     return LBMOE_OK;
   }
-  if (!rt && use_tiled(L, gw, x, T, k)) {
+  if (!rt && use_tiled(L, gw, T, k)) {
     // prefill-sized batch: LDS-tiled MFMA GEMMs over a device-built token-tile list
     if (!tiles_built)
       LBMOE_TRY(launch_build_tiles(counts, offsets, gw, with_shared, T, max_tiles, tiles, s));
@@ -417,11 +424,11 @@ struct NormArgs {
 
 // Whether the block routes through launch_router_route: the tiled router over at most 128
 // experts, with the tiled expert GEMMs after it (their tile list is built with the scatter).
-static bool route_in_router(const lbmoe_layer& L, const void* x, int64_t T, bool sh) {
+static bool route_in_router(const lbmoe_layer& L, int64_t T, bool sh) {
   const int E = L.num_experts, H = L.hidden_size, k = L.top_k;
   if (!router_is_tiled(T, E, H) || !router_route_supported(E, H, k)) return false;
   const GroupWeights gw = group_weights(L, sh, T);
-  if (!use_tiled(L, gw, x, T, k)) return false;
+  if (!use_tiled(L, gw, T, k)) return false;
   return !is_fp8(L) || tiled_fp8_supported(gw, T, T * k + (sh ? T : 0));
 }
 
@@ -446,7 +453,7 @@ static int32_t forward_impl(const lbmoe_layer* layer, const void* x, int64_t T, 
   float* sgate = sh ? at<float>(ws, w, R_SGATE) : nullptr;
   LBMOE_TRY(ev->mark(s));
   void* xn = norm ? at<void>(ws, w, R_XN) : nullptr;     // the norm's output: the block's input
-  if (route_in_router(L, norm ? xn : x, T, sh)) {
+  if (route_in_router(L, T, sh)) {
     // the norm's own kernel first (1024 tokens or more: the router would recompute it per tile);
     // the norm path then saves the same launches as the plain one, Qwen3-30B-A3B T=1024 267.5 -> 264.1
     // us, H = 1024 E = 16 T=2048 70.4 -> 69.5
@@ -479,7 +486,7 @@ static int32_t forward_impl(const lbmoe_layer* layer, const void* x, int64_t T, 
   }
   LBMOE_TRY(ev->mark(s));
   const GroupWeights gw = group_weights(L, sh, T);
-  const bool streams = !is_fp8(L) && !use_tiled(L, gw, x, T, L.top_k);   // the bf16 decode GEMMs
+  const bool streams = !is_fp8(L) && !use_tiled(L, gw, T, L.top_k);   // the bf16 decode GEMMs
   // the smallest bf16 batches route inside the gate_up kernel (profiled calls then have
   // empty routing and permutation stages)
   if (streams && inline_route_supported(T, L.top_k, L.num_experts)) {
@@ -706,7 +713,7 @@ int32_t lbmoe_dense_mlp(const void* gate_proj, const void* up_proj, const void* 
     LBMOE_TRY(launch_down_fp8(gw, actq, acts, Imax, nullptr, nullptr, T, 1, out, s));
     return LBMOE_OK;
   }
-  if (dense_tiled_supported(gw, x, T, Imax, act, out)) {
+  if (dense_tiled_supported(gw, T, Imax, act, out)) {
     LBMOE_TRY(launch_dense_tiled(gw, x, T, Imax, act, out, s));
     return LBMOE_OK;
   }

@@ -263,14 +263,15 @@ hipError_t launch_down_tiled_fp8(const GroupWeights& gw, const void* actq, const
                                  int act_ld, const int32_t* tiles, int max_tiles, void* out,
                                  hipStream_t s);
 // The dense MLP on LDS-tiled GEMMs (weights gw.sh_*, act rows act_ld apart): batches of at least
-// kDenseTiledMinTokens tokens with 16-byte aligned operands within the buffer copies' range. Up to
-// 28 tokens the streaming kernels run two token tiles per pass (H = 2048, Is = 512: T=24 9.4 us
-// against 11.4), above four (T=32 12.4 against 11.5). A tile shape is taken where it gives at least
+// kDenseTiledMinTokens tokens with weights, workspace and output on 16-byte boundaries, operands within
+// the buffer copies' range. Up to 28 tokens the streaming kernels run two token tiles per pass (H = 2048,
+// Is = 512: T=24 9.4 us against 11.4), above four (T=32 12.4 against 11.5). Weights 2 bytes off cost
+// the tiles of small batches more (T=200 14.2 / 18.3), token rows anywhere do not (17.8 / 16.9). A tile shape is taken where it gives at least
 // kDenseMinWorkgroups workgroups (launch_dense_gemm).
 constexpr int64_t kDenseTiledMinTokens = 29;
 constexpr int64_t kDenseMinWorkgroups = 160;
-bool dense_tiled_supported(const GroupWeights& gw, const void* x, int64_t T, int act_ld,
-                           const void* act, const void* out);
+bool dense_tiled_supported(const GroupWeights& gw, int64_t T, int act_ld, const void* act,
+                           const void* out);
 hipError_t launch_dense_tiled(const GroupWeights& gw, const void* x, int64_t T, int act_ld,
                               void* act, void* out, hipStream_t s);
 // fp8: xq, xs are x's codes and scales; gate_up writes the act's.
@@ -281,10 +282,11 @@ hipError_t launch_dense_tiled_fp8(const GroupWeights& gw, const void* xq, const 
                                   hipStream_t s);
 bool tiled_router_supported(int E, int H);
 // whether launch_router_logits_tiled takes 64 x 64 tiles with the k range split
-bool router_small_tiles(const void* x, const void* wg, const void* logits, int64_t T, int E,
-                        int H);
-// Whether every pointer is 16-byte aligned, as the direct global -> LDS copies and whole-row
-// stores of the tiles that callers' tensors reach are kept.
+bool router_small_tiles(const void* logits, int64_t T, int E, int H);
+// Whether every pointer is 16-byte aligned. The direct global -> LDS copies of the tiled kernels take
+// operands at any address, with the same results (the memory side of a buffer access may be unaligned
+// on this target); what is kept to boundaries are the weights where an unaligned stream costs more
+// than the other kernels, and the whole-row stores into callers' tensors.
 inline bool aligned16(std::initializer_list<const void*> ptrs) {
   uintptr_t bits = 0;
   for (const void* p : ptrs) bits |= reinterpret_cast<uintptr_t>(p);

@@ -307,7 +307,7 @@ bool router_is_tiled(int64_t T, int E, int H) {
 
 hipError_t launch_router_logits(const void* x, const void* wg, int64_t T, int E, int H,
                                 void* logits, hipStream_t s) {
-  if (router_is_tiled(T, E, H) || router_small_tiles(x, wg, logits, T, E, H))
+  if (router_is_tiled(T, E, H) || router_small_tiles(logits, T, E, H))
     return launch_router_logits_tiled(x, wg, T, E, H, logits, s);
   return launch_router_decode<false>(static_cast<const uint16_t*>(x), NormIn{}, wg, T, E, H,
                                      logits, s);

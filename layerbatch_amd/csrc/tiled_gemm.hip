@@ -1522,10 +1522,10 @@ static hipError_t launch_dense_gemm(const GroupWeights& gw, const void* src, int
   return launch_dense_small<MODE>(gw, K, src, src_ld, T, dst, dst_ld, s);
 }
 
-bool dense_tiled_supported(const GroupWeights& gw, const void* x, int64_t T, int act_ld,
-                           const void* act, const void* out) {
+bool dense_tiled_supported(const GroupWeights& gw, int64_t T, int act_ld, const void* act,
+                           const void* out) {
   return T >= kDenseTiledMinTokens && bf16_tiled_offsets_fit(T, 0, gw.H, act_ld) &&
-         aligned16({x, act, out, gw.sh_gate, gw.sh_up, gw.sh_down});
+         aligned16({act, out, gw.sh_gate, gw.sh_up, gw.sh_down});
 }
 
 hipError_t launch_dense_tiled(const GroupWeights& gw, const void* x, int64_t T, int act_ld,
@@ -1671,11 +1671,11 @@ hipError_t launch_perm_scatter_build(const void* idx, int idx_bytes, int64_t T, 
 // tiles fit the CUs at once. Measured with the selection (us, E = 512 / 128, H = 2048): T=128
 // streaming 9.2 / 8.5, these 10.8 / 10.2; T=256 12.7 / 8.7 and 10.9 / 10.2; T=777 32.3 / 10 and
 // 11.2 / 10.2; T=1024 15.4 / 14.7 (128 x 64 tiles of whole k) and 11.4 / 10.3; T=2048 16.5 / 15.0
-// and 12.9 / 10.7; T=4096 19.4 / 16.0 and 23.6 / 11.8; T=8192 30.4 / 17.9 and 42.3 / 16.2.
+// and 12.9 / 10.7; T=4096 19.4 / 16.0 and 23.6 / 11.8; T=8192 30.4 / 17.9 and 42.3 / 16.2. Token rows
+// or weights 2 bytes off a 16-byte boundary, the logits alone: E = 512, T=777 61 / 12.6 and 63 / 12.8.
 constexpr int64_t kStreamRouterMaxTiles = 384;
-bool router_small_tiles(const void* x, const void* wg, const void* logits, int64_t T, int E,
-                        int H) {
-  return tiled_router_supported(E, H) && T * H * 2 < kTiledMaxBytes && aligned16({x, wg, logits}) &&
+bool router_small_tiles(const void* logits, int64_t T, int E, int H) {
+  return tiled_router_supported(E, H) && T * H * 2 < kTiledMaxBytes && aligned16({logits}) &&
          static_cast<int64_t>((E + 15) / 16) * ((T + 15) / 16) > kStreamRouterMaxTiles &&
          (T + 63) / 64 * ((E + 63) / 64) <= device_cus();
 }
@@ -1716,7 +1716,7 @@ hipError_t launch_router_logits_tiled(const void* x, const void* wg, int64_t T, 
   gw.gate_up = wg;
   gw.E = E;
   gw.H = H;
-  if (router_small_tiles(x, wg, logits, T, E, H))
+  if (router_small_tiles(logits, T, E, H))
     return launch_dense_small<kRouter>(gw, H, x, H, T, logits, E, s);
   if (E <= RouterShape128::kRows) return launch_router_shape<RouterShape128>(gw, x, T, logits, s);
   const int64_t tall = (T + RouterShapeTall::kWT - 1) / RouterShapeTall::kWT *

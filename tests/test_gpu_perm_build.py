@@ -88,9 +88,17 @@ def test_fp8_block_at_the_switch(gpu, shape, T):
     _run_fp8(shape, T, gpu, seed=T, sample=48)
 
 
+def _at(t, off):
+    """t's values in a tensor that starts off bytes past a 16-byte boundary."""
+    n = t.numel() * t.element_size()
+    v = torch.empty(n + 32, dtype=torch.uint8, device=t.device)[off:off + n].view(t.dtype).view(t.shape)
+    v.copy_(t)
+    assert v.data_ptr() % 16 == off
+    return v
+
+
 def test_unaligned_rows_at_the_switch(gpu):
-    """Token rows between 16-byte boundaries: the same result (below 28 tokens per expert they stay
-    on the streaming kernels)."""
+    """Token rows between 16-byte boundaries: the same result."""
     shape, T = MoEShape(256, 256, 4, 256, 0), 1024
     w, g = make_layer(shape, seed=4)
     blk = _block(shape, {n: v.to(gpu) for n, v in w.items()}, gpu)
@@ -101,3 +109,54 @@ def test_unaligned_rows_at_the_switch(gpu):
     # a router logit summed in another order may move a token to another expert: all but a few rows
     close = np.abs(a - b).max(axis=1) <= gc.TOL_BF16 * np.abs(a).max()
     assert close.mean() >= 0.99
+
+
+# T = 1100: 17 tokens per expert, where weights between 16-byte boundaries stay on the streaming
+# kernels; 3000: 47, copies from any address. Wide, narrow and tiny tiles. The same indices on both sides, so
+# that one kernel's results do not depend on the addresses by a bit
+@pytest.mark.parametrize("T", [1100, 3000])
+@pytest.mark.parametrize("what,fp8", [("x", False), ("workspace", False), ("weights", False),
+                                      ("packed", False), ("x", True), ("workspace", True),
+                                      ("weights", True)])
+def test_operands_between_boundaries(gpu, T, what, fp8):
+    shape, k = MoEShape(512, 256, 4, 256, 256), 4
+    w, g = make_layer(shape, seed=6)
+    x = make_x(g, T, 512).to(gpu)
+    blk = _block(shape, {n: v.to(gpu) for n, v in w.items()}, gpu)
+    if fp8:
+        blk.quantize_fp8_()
+    elif what == "packed":
+        blk.pack_tiled_()
+    ex = blk.experts
+    idx = 2 + torch.rand((T, 254), generator=g).argsort(dim=1)[:, :k]
+    idx[:T // 2, 0], idx[T // 2:T // 2 + 100, 0] = 0, 1       # experts of T / 2 and of 100 tokens
+    idx = idx.to(gpu, torch.int32).contiguous()
+    tw = torch.rand((T, k), generator=g).to(gpu, torch.bfloat16)
+
+    def run(off):
+        L = _lib.LbmoeLayer()
+        ex.fill_layer(L)
+        L.top_k = k
+        n = _lib.workspace_size(L, T)
+        ws = torch.empty(n + 32, dtype=torch.uint8, device=gpu)[(off if what == "workspace" else 0):][:n]
+        y = torch.empty_like(x)
+        xv = _at(x, off) if what == "x" else x
+        _lib.check(_lib.lib().lbmoe_experts(
+            ctypes.byref(L), _lib.ptr(xv), _lib.ptr(idx), 4, _lib.ptr(tw), T, _lib.ptr(y), _lib.ptr(ws),
+            ws.numel(), _lib.stream_of(gpu)), "lbmoe_experts")
+        torch.cuda.synchronize()
+        return y
+
+    want = run(0)
+    for off in (2, 4, 8) if what in ("x", "packed") else (4, 12) if what == "workspace" else (8, 2):
+        if what == "weights" and fp8:
+            ex.gate_up_q, ex.down_q = _at(ex.gate_up_q, off - 1), _at(ex.down_q, off - 1)
+        elif what == "weights":
+            ex.gate_up_proj.data, ex.down_proj.data = _at(ex.gate_up_proj.data, off), _at(ex.down_proj.data, off)
+        elif what == "packed":
+            ex.gate_up_tiled, ex.down_tiled = _at(ex.gate_up_tiled, off), _at(ex.down_tiled, off)
+        got = run(off)
+        if T < 28 * 256 // k and what in ("weights", "packed") and not fp8:
+            gc.check_output(to_np(got), to_np(want).astype("float64"), gc.TOL_BF16)   # other kernels
+        else:
+            assert torch.equal(got, want)
