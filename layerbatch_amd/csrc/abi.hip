@@ -166,6 +166,11 @@ static P* at(void* ws, const WsLayout& w, int r) {
     if ((expr) != hipSuccess) return LBMOE_ERR_LAUNCH;        \
   } while (0)
 
+static CallSizes call_sizes(const lbmoe_layer& L, bool with_shared, int64_t T) {
+  return {L.num_experts, L.hidden_size, L.moe_intermediate_size,
+          with_shared ? L.shared_intermediate_size : 0, T, is_fp8(L), device_cus()};
+}
+
 // Whether the call's experts run on the LDS-tiled GEMMs (tiled_min_tokens). Their copies take operands
 // at any address, but weights between 16-byte boundaries cost them more than the streaming kernels, so
 // those leave the latter from kTiledAlways only (Qwen3-30B-A3B, us streaming / tiled: T = 256 weights 8
@@ -176,8 +181,7 @@ static bool use_tiled(const lbmoe_layer& L, const GroupWeights& gw, int64_t T, i
   const double avg = static_cast<double>(T) * k / gw.E;
   if (avg >= kTiledAlways) return true;
   const bool sh = gw.groups > gw.E;
-  const CallSizes c{gw.E, gw.H, gw.I, sh ? gw.Is : 0, T, is_fp8(L), device_cus()};
-  if (avg < tiled_min_tokens(c)) return false;
+  if (avg < tiled_min_tokens(call_sizes(L, sh, T))) return false;
   auto copied = [](const void* packed, const void* w) { return packed ? packed : w; };
   return aligned16({copied(gw.gate_up_tiled, gw.gate_up), copied(gw.down_tiled, gw.down)}) &&
          (!sh || aligned16({copied(gw.sh_gate_up_tiled, gw.sh_gate),
@@ -489,7 +493,8 @@ static int32_t forward_impl(const lbmoe_layer* layer, const void* x, int64_t T, 
   const bool streams = !is_fp8(L) && !use_tiled(L, gw, T, L.top_k);   // the bf16 decode GEMMs
   // the smallest bf16 batches route inside the gate_up kernel (profiled calls then have
   // empty routing and permutation stages)
-  if (streams && inline_route_supported(T, L.top_k, L.num_experts)) {
+  if (streams && inline_route_supported(T, L.top_k, L.num_experts) &&
+      route_in_gate_up_pays(call_sizes(L, sh, T), L.top_k)) {
     const SmallRoute rt{static_cast<const uint16_t*>(logits), L.logit_bias,
                         static_cast<const uint16_t*>(L.shared_expert_gate), L.top_k,
                         static_cast<int32_t*>(idx), static_cast<uint16_t*>(topw), sgate,

@@ -159,9 +159,9 @@ hipError_t launch_gate_up_bf16(const GroupWeights& gw, const void* x, const int3
 // Batches of at most kInlineRouteTokens tokens (and T*k <= kInlineRouteEntries) skip the
 // route and permutation kernels on the bf16 decode path: every gate_up workgroup selects the
 // batch's experts from the logits itself (launch_gate_up_bf16_routed) and derives its own
-// group's rows, and the workgroups of the first channel block store the routing outputs. With 5 to
-// 8 tokens each of a workgroup's four waves selects up to two, still less than the launch it saves
-// (E = 64, T=5 30.0 -> 27.5 us per layer, E = 96 top-3 T=8 28.5 -> 25.9, Qwen3-30B-A3B T=5..8 0.2-1%).
+// group's rows, and the workgroups of the first channel block store the routing outputs. With more
+// than 4 tokens only while a CU runs few of them (route_in_gate_up_pays: E = 64, T=5 30.0 -> 27.5 us
+// per layer, E = 96 top-3 T=8 28.5 -> 25.9).
 constexpr int64_t kInlineRouteTokens = 8;
 constexpr int kInlineRouteEntries = 64;
 bool inline_route_supported(int64_t T, int k, int E);

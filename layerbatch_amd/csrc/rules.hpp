@@ -69,4 +69,21 @@ inline double tiled_min_tokens(const CallSizes& c) {
   return std::clamp(t, 8.0, kTiledAlways);
 }
 
+// Whether a batch that fits (kInlineRouteTokens, kInlineRouteEntries) is better routed inside the
+// bf16 decode gate_up kernel, by every workgroup for itself, than by a launch of its own. Up to 4
+// tokens always: a wave selects one token. With 5 to 8 each wave selects up to two, which a CU repeats
+// for every workgroup it runs, and more experts per lane hold more registers, so fewer workgroups are
+// resident: the more of them per CU, the more of the saved launch goes. Measured (us per layer,
+// separate / inside) around the lines:
+//   E <= 256: 5 per CU 43.8 / 42.9, 7.5 71.8 / 71.1 and 33.8 / 33.3, 8 81.7 / 79.7; 8.1 55.5 / 57.2,
+//     9 35.7 / 38.0, 10.5 49.7 / 51.9, 12 40.1 / 43.4
+//   E <= 512: 2.5 31.1 / 28.2, 4 36.4 / 34.2; 4.6 51.7 / 56.1, 5 30.2 / 31.2, 8 36.1 / 39.4
+//   E > 512: 2 30.9 / 29.7, 3 48.6 / 46.9; 3.1 37.7 / 41.3, 3.5 38.9 / 42.2, 7 79.0 / 83.9
+inline bool route_in_gate_up_pays(const CallSizes& c, int k) {
+  if (c.T <= 4) return true;
+  const int64_t rows = std::min<int64_t>(c.T * k, c.E) + (c.Is > 0 ? 1 : 0);
+  const int64_t per_cu = c.E <= 256 ? 8 : c.E <= 512 ? 4 : 3;
+  return std::max(c.I, c.Is) / 16 * rows <= per_cu * c.cus;
+}
+
 }  // namespace lbmoe

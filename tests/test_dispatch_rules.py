@@ -62,6 +62,28 @@ def test_tiled_line_takes_the_measured_side(tmp_path):
         assert (T * 8 / E >= line) == (tiled < stream), (H, E, I, Is, T, fp8, line)
 
 
+# H, E, k, I, Is, T, us with a routing launch, us routed inside gate_up
+MEASURED_ROUTE = [
+    (1024, 20, 3, 512, 0, 8, 25.3, 23.6), (1024, 256, 10, 256, 256, 6, 36.9, 33.7),
+    (1536, 64, 10, 384, 0, 5, 41.9, 39.9), (2048, 160, 9, 512, 256, 7, 81.7, 79.7),
+    (1024, 256, 8, 512, 256, 8, 55.5, 57.2), (512, 160, 8, 768, 0, 6, 35.7, 38.0),
+    (512, 100, 12, 768, 0, 5, 37.8, 41.8), (1024, 512, 4, 512, 0, 8, 36.4, 34.2),
+    (2048, 512, 8, 256, 0, 8, 55.8, 53.4), (1536, 512, 7, 384, 0, 6, 45.2, 42.8),
+    (1536, 512, 7, 384, 0, 7, 51.7, 56.1), (512, 512, 8, 512, 0, 5, 30.2, 31.2),
+    (1024, 1000, 8, 256, 0, 6, 36.5, 34.8), (1024, 1000, 8, 256, 0, 7, 38.9, 42.2),
+    (2048, 1000, 3, 512, 0, 8, 48.6, 46.9), (1024, 1000, 6, 256, 256, 8, 37.7, 41.3),
+    (2048, 1024, 8, 512, 0, 8, 86.1, 91.8),
+]
+
+
+def test_routing_inside_gate_up_takes_the_measured_side(tmp_path):
+    got = _evaluate(tmp_path, [
+        f"route_in_gate_up_pays(CallSizes{{{E}, {H}, {I}, {Is}, {T}, false, 256}}, {k})"
+        for H, E, k, I, Is, T, _, _ in MEASURED_ROUTE])
+    for case, inside in zip(MEASURED_ROUTE, got):
+        assert bool(inside) == (case[-1] < case[-2]), case
+
+
 @pytest.mark.parametrize("E,I", [(16, 512), (4, 768), (1, 256)])
 def test_few_items_stay_on_the_streaming_kernels(tmp_path, E, I):
     sizes = [f"CallSizes{{{E}, 2048, {I}, {Is}, 50, {fp8}, 256}}" for Is in (0, 512)
