@@ -457,10 +457,8 @@ static int32_t forward_impl(const lbmoe_layer* layer, const void* x, int64_t T, 
   float* sgate = sh ? at<float>(ws, w, R_SGATE) : nullptr;
   LBMOE_TRY(ev->mark(s));
   void* xn = norm ? at<void>(ws, w, R_XN) : nullptr;     // the norm's output: the block's input
-  if (route_in_router(L, T, sh)) {
-    // the norm's own kernel first (1024 tokens or more: the router would recompute it per tile);
-    // the norm path then saves the same launches as the plain one, Qwen3-30B-A3B T=1024 267.5 -> 264.1
-    // us, H = 1024 E = 16 T=2048 70.4 -> 69.5
+  if (route_in_router(L, T, sh) && (!norm || norm_takes_selecting_router(call_sizes(L, sh, T)))) {
+    // the norm's own kernel first (1024 tokens or more: the router would recompute it per tile)
     if (norm) {
       LBMOE_TRY(launch_add_rmsnorm(x, norm->residual, norm->weight, norm->eps, T, L.hidden_size, xn,
                                    norm->residual_out, s));

@@ -86,4 +86,15 @@ inline bool route_in_gate_up_pays(const CallSizes& c, int k) {
   return std::max(c.I, c.Is) / 16 * rows <= per_cu * c.cus;
 }
 
+// Whether a batch behind the residual add and RMSNorm takes the router that also selects (where the
+// plain block does, route_in_router). Behind the norm's own kernel the plain router and the selection
+// of their own cost as many launches more as without it, but the selecting router's workgroups each
+// compute the shared expert's gate of 64 tokens one after another, and at short rows its launch is
+// little shorter (us, plain router / selecting: Qwen3-30B-A3B T=1024 267.5 / 264.1; I = 256: H = 2048,
+// E = 96, k = 1, T=4096 with a shared expert of 512 145.5 / 155.4, without one T=6000 135 / 140,
+// T=8192 169 / 166; E = 48, k = 4, T=1500 103.5 / 98.7; H = 1024, E = 64, k = 1, shared, T=3000 80.4 /
+// 86.1; H = 512, E = 16, k = 2, T=1024 46.2 / 48.5, T=8192 65.7 / 65.3; H = 1024 without a shared
+// expert within 2% either way).
+inline bool norm_takes_selecting_router(const CallSizes& c) { return c.Is == 0 && c.H >= 1024; }
+
 }  // namespace lbmoe

@@ -84,6 +84,23 @@ def test_routing_inside_gate_up_takes_the_measured_side(tmp_path):
         assert bool(inside) == (case[-1] < case[-2]), case
 
 
+# H, E, k, Is, T (I = 256), us with the plain router behind the norm, us with the selecting one
+MEASURED_NORM = [
+    (2048, 96, 1, 512, 4096, 145.5, 155.4), (1024, 64, 1, 512, 3000, 80.4, 86.1),
+    (512, 64, 1, 512, 2048, 57.9, 62.8), (512, 16, 2, 0, 1024, 46.2, 48.5),
+    (2048, 128, 2, 512, 2048, 137.5, 144.1), (2048, 48, 4, 0, 1500, 103.5, 98.7),
+    (2048, 16, 2, 0, 1500, 84.4, 81.0), (2048, 128, 8, 0, 1024, 127.5, 122.9),
+]
+
+
+def test_norm_path_takes_the_measured_router(tmp_path):
+    got = _evaluate(tmp_path, [
+        f"norm_takes_selecting_router(CallSizes{{{E}, {H}, 256, {Is}, {T}, false, 256}})"
+        for H, E, _, Is, T, _, _ in MEASURED_NORM])
+    for case, selecting in zip(MEASURED_NORM, got):
+        assert bool(selecting) == (case[-1] < case[-2]), case
+
+
 @pytest.mark.parametrize("E,I", [(16, 512), (4, 768), (1, 256)])
 def test_few_items_stay_on_the_streaming_kernels(tmp_path, E, I):
     sizes = [f"CallSizes{{{E}, 2048, {I}, {Is}, 50, {fp8}, 256}}" for Is in (0, 512)

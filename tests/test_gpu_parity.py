@@ -451,21 +451,24 @@ def test_forward_norm(gpu, shape_name, T):
 
 
 # T >= 1024 with at most 128 experts on the tiled GEMMs: the norm's own kernel, then the router that
-# also selects (k range split over workgroups, or from 16384 tokens whole), which reads the normalised
-# rows for the logits and for the shared expert's gate
+# also selects (H >= 1024 without a shared expert: k range split over workgroups, or from 16384 tokens
+# whole) or the plain one and the selection, which reads the normalised rows for the shared expert's gate
 @pytest.mark.parametrize("shape,T,fp8", [
     (SHAPES["small-h1024-e16"], 1100, False), (SHAPES["qwen3-30b-a3b"], 1024, False),
+    (MoEShape(1024, 64, 4, 256, 0), 1501, False), (MoEShape(1024, 32, 2, 256, 0), 1300, True),
+    (MoEShape(1024, 20, 2, 256, 0), 16391, False), (MoEShape(1024, 64, 4, 256, 256), 1501, False),
     (MoEShape(512, 64, 4, 256, 256), 1501, False), (MoEShape(512, 32, 2, 256, 256), 1300, True),
     (MoEShape(512, 20, 2, 256, 128), 16391, False)])
 def test_forward_norm_fused_router(gpu, shape, T, fp8):
-    _check_forward_norm(gpu, shape, T, fp8)
+    selecting = shape.hidden_size >= 1024 and not shape.shared_expert_intermediate_size
+    _check_forward_norm(gpu, shape, T, fp8, same_router=selecting)
 
 
-def _check_forward_norm(gpu, shape, T, fp8=False):
+def _check_forward_norm(gpu, shape, T, fp8=False, same_router=True):
     """Residual add + RMSNorm + block (qwen3_5.py:998-1004): the new residual is the bf16 sum
     bit for bit, the block input within one bf16 step of the oracle's Qwen3_5RMSNorm, and the
-    output equals the plain block on that input bit for bit (decode T: norm fused into the
-    router kernel; more tokens: separate norm kernel)."""
+    output equals the plain block on that input bit for bit where both take one router (decode T:
+    norm fused into the router kernel; more tokens: separate norm kernel)."""
     H = shape.hidden_size
     w, g = make_layer(shape, seed=T, device=gpu)
     blk = _block(shape, w, gpu)
@@ -482,9 +485,26 @@ def _check_forward_norm(gpu, shape, T, fp8=False):
     xn = _region(blk, ws, T, "xn", torch.bfloat16, (T, H)).clone()
     d = np.abs(bf16_bits_of(xn).astype(np.int32) - bf16_bits(x_ref).astype(np.int32))
     assert d.max() <= 1, f"block input differs from the oracle's RMSNorm by {d.max()} bf16 steps"
-    y_plain = blk(xn)
+    ws2 = torch.empty_like(ws)
+    y_plain = blk(xn, workspace=ws2)
     torch.cuda.synchronize()
-    assert torch.equal(y, y_plain)
+    if same_router:
+        assert torch.equal(y, y_plain)
+        return
+    # the plain block's router sums the logits in another order: both selections follow their own
+    # logits, and the rows that got the same experts and weights agree
+    k, E = shape.top_k, shape.num_experts
+    logits, idx, topw = (_region(blk, ws, T, *r) for r in (
+        ("logits", torch.bfloat16, (T, E)), ("topk_idx", torch.int32, (T, k)),
+        ("topk_w", torch.bfloat16, (T, k))))
+    rows = np.arange(0, T, max(1, T // 500))
+    gc.check_logits(bf16_bits_of(logits)[rows], to_np(xn)[rows], to_np(w["gate"]))
+    gc.check_route(to_np(idx), bf16_bits_of(topw), to_np(logits), None, k)
+    same = ((idx == _region(blk, ws2, T, "topk_idx", torch.int32, (T, k))).all(dim=1)
+            & (topw == _region(blk, ws2, T, "topk_w", torch.bfloat16, (T, k))).all(dim=1))
+    assert same.float().mean() > 0.9
+    gc.check_output(to_np(y[same]), to_np(y_plain[same]).astype("float64"),
+                    gc.TOL_FP8 if fp8 else gc.TOL_BF16)
 
 
 def test_forward_norm_rejects_in_place_residual(gpu, lbmoe):
