@@ -697,12 +697,18 @@ __device__ __forceinline__ void tile_product(const GroupWeights& gw, const uint1
   // 128 bytes of every 4 KB row at about the same time, which lands on few HBM channels, how few
   // depending on where the weights were allocated: Qwen3-30B-A3B experts T=509 221-254 us by
   // allocation, rotated 209; T=512 layer 235-266 -> 220, T=2048 333-345 -> 322, E=512 T=4096 703 ->
-  // 692. Wide tiles stay in step: they share operands through L2 (T=8192 uniform 744 -> 768 us
+  // 692; under a Zipf bias T=8192, 4096 and 2048 are level (723 / 720, 421 / 421, 280 / 279). Narrow
+  // tiles keep k = 0 below 12 k-tiles in gate_up and 8 in down: there is little to gain from short rows,
+  // and down at I = 256 lost (E = 128, H = 512, 1024, 1536, T=2560 46.5 -> 48.8, 68.7 -> 71.6, 91.6 ->
+  // 95.5; I = 512, E = 512, H = 1024, T=8192 340 -> 326; I = 768, E = 128 149 -> 145), gate_up at H =
+  // 512 by 1.5%. Wide tiles stay in step: they share operands through L2 (T=8192 uniform 744 -> 768 us
   // rotated), and the fp8 tiles, with half the bytes per row, gain nothing (E=512 T=4096 477 -> 480).
   constexpr bool kRotate = !ROUTER && !DENSE && S::kWT < kWM;
-  const int rot = kRotate ? static_cast<int>((5u * static_cast<uint32_t>(wt) + 3u * static_cast<uint32_t>(g)) %
-                                             static_cast<uint32_t>(nk))
-                          : 0;
+  constexpr int kRotateMinTiles = S::kWT == 64 ? 1 : GATEUP ? 12 : 8;
+  const int rot = kRotate && nk >= kRotateMinTiles
+                      ? static_cast<int>((5u * static_cast<uint32_t>(wt) + 3u * static_cast<uint32_t>(g)) %
+                                         static_cast<uint32_t>(nk))
+                      : 0;
   auto k_of = [&](int kt) {                   // k-tile of the matrix at step kt of the product
     if constexpr (!kRotate) return kt;
     const int r = kt + rot;
