@@ -264,10 +264,17 @@ hipError_t launch_down_tiled_fp8(const GroupWeights& gw, const void* actq, const
                                  hipStream_t s);
 // The dense MLP on LDS-tiled GEMMs (weights gw.sh_*, act rows act_ld apart): batches of at least
 // kDenseTiledMinTokens tokens with weights, workspace and output on 16-byte boundaries, operands within
-// the buffer copies' range. Up to 28 tokens the streaming kernels run two token tiles per pass (H = 2048,
-// Is = 512: T=24 9.4 us against 11.4), above four (T=32 12.4 against 11.5). Weights 2 bytes off cost
-// the tiles of small batches more (T=200 14.2 / 18.3), token rows anywhere do not (17.8 / 16.9). A tile shape is taken where it gives at least
-// kDenseMinWorkgroups workgroups (launch_dense_gemm).
+// the buffer copies' range. Up to 28 tokens the streaming kernels run two token tiles per pass (H =
+// 2048, Is = 512: T=24 9.4 us against 11.4), above four (T=32 12.4 against 11.5). From 29 on the tiles
+// won or were level at every size measured with the weights in HBM (H = 512 to 2048, Is = 128 to 3072, T
+// up to 8192; streaming / tiles at T=29: H = 512, Is = 256 8.4 / 7.8, H = 2048, Is = 2048 21.9 / 18.8;
+// fp8, whose gate_up then runs on two workgroups at Is = 256, 24.4 / 20.4 at H = 2048 and 13.6 / 12.3 at
+// H = 512). Weights 2 bytes off cost the tiles of small batches more (T=200 14.2 / 18.3), token rows
+// anywhere do not (17.8 / 16.9).
+// A tile shape is taken where it gives at least kDenseMinWorkgroups workgroups (launch_dense_gemm): of
+// 80, 110, 160 and 256 the best over H = 512 to 2048, Is = 256 to 768, T = 200 to 8192 (geometric mean
+// over the best of each size 1.13, 1.04, 1.04 and 1.12, in fp8 1.10, 1.05, 1.01 and 1.02; at worst, where
+// the workgroups end just past a whole round, 1.39: H = 1536, Is = 768, T=700 26.3 against 18.9 with 110).
 constexpr int64_t kDenseTiledMinTokens = 29;
 constexpr int64_t kDenseMinWorkgroups = 160;
 bool dense_tiled_supported(const GroupWeights& gw, int64_t T, int act_ld, const void* act,
