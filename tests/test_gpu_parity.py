@@ -588,8 +588,9 @@ def test_router_logits_tiled_shapes(gpu, E, T):
 
 
 # small batches (up to 16 tokens for E <= 128, up to 4 otherwise) route and permute in one
-# kernel (one wave per token, then the one-workgroup permutation), and up to 4 tokens with
-# T*k <= 64 inside every gate_up workgroup instead (bf16): every expert-count class of the
+# kernel (one wave per token, then the one-workgroup permutation), and up to 4 tokens (8 with few
+# gate_up workgroups) with T*k <= 64 inside every gate_up workgroup instead (bf16), or with at least
+# as many pairs as experts permute inside it: every expert-count class of the
 # route, with and without a shared expert, with the compact workgroup rows (T*k < E) and
 # without them, and batches just past the limits; the routing regions are checked too
 @pytest.mark.parametrize("shape,T", [(MoEShape(512, 1024, 10, 256, 0), 4),
