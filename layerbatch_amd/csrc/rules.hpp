@@ -19,31 +19,35 @@ struct CallSizes {
 
 // Tokens per routed expert from which the LDS-tiled GEMMs replace weight streaming. The streaming
 // kernels run two token tiles per pass above 8 tokens per expert and four above 28 (kTiledAlways),
-// each step slower; the tiled ones barely depend on the count, but a launch takes whole rounds of the
-// CUs (one workgroup each), so what counts is
+// each step slower, and walk a popular expert's rows pass after pass; the tiled ones barely depend on
+// the counts, but a launch takes whole rounds of the CUs (one workgroup each). So what counts in bf16 is
 //   - the share of the last round that idles: gate_up's items are one per expert and 128
 //     intermediate channels, the shared expert's one per 256 tokens and 128 channels, and two of
-//     those past a whole number of rounds cost a round (bf16 H = 2048, E = 64, I = Is = 512, 13
-//     tokens: streaming 91 us, tiled 114; without the shared expert 84 / 85);
+//     those past a whole number of rounds cost a round (H = 2048, E = 64, I = Is = 512, 13 tokens:
+//     streaming 91 us, tiled 114; without the shared expert 84 / 85);
 //   - down's (rows of 256 output channels, cheaper items);
 //   - a launch of less than one round, whose length is its longest item's;
-//   - for fp8, a shared expert (its wide item then holds up a short launch) and short k ranges (H =
-//     512: four k-tiles per item);
 //   - a shared expert wider than the routed ones: the streaming launches' workgroups are laid out by
 //     the wider of the two, the routed ones past their own width idle (H = 2048, E = 512, I = 256, Is
-//     = 512, 8 tokens: 416 / 316).
-// The weights come from 3036 layer calls timed both ways (GPU us, in turn in one process; E = 32..512, I =
-// 128..768, Is = 0, 256, 512, H = 512, 1024, 2048, 8 to 27 tokens per expert, uniform routing): the
-// side taken is slower than the other by more than 3% in 2% of the bf16 and 6% of the fp8 calls, and
-// slower than streaming by more than 3% in 0.5% and 2%, at worst 9%. A line by the routed items
-// alone lost more than 3% to streaming in 6% and 15%, up to 25%.
-// Skewed routings gain from the tiled kernels earlier: under a Zipf bias the streaming kernels walk a
-// popular expert's rows pass after pass (E = 512, 7.5 tokens: 477 / 139).
+//     = 512, 8 tokens: 416 / 316);
+//   - the experts: the more there are, the more of a skewed routing's rows lie with few of them. Under
+//     a Zipf bias tiled takes 0.9 of streaming's time at E = 32 and 13 tokens per expert, 0.6 at 128,
+//     0.3 at 512 (Qwen3-30B-A3B with a shared expert, 13 tokens: 142 / 66 us).
+// The host cannot see the skew. The weights come from 5420 layer calls timed both ways (GPU us, in turn
+// in one process; E = 32..512, I = 128..768, Is = 0, 256, 512, H = 512, 1024, 2048, 8 to 27 tokens per
+// expert), for the least expected log time with three uniform calls to one under a Zipf bias: uniform
+// calls then lie 0.6% above the faster side, more than 3% above streaming in 2% of the cases, at worst
+// 10%. By the routed experts' items alone they lay 1.4% above it, at worst 25% above streaming, and the
+// calls under a bias 4% higher.
+// fp8 (its streaming kernels stream less per wave) gains more from the tiles under a bias, 0.8 at E = 32
+// and 0.25 at 512 and 10 tokens per expert, against up to 16% on uniform calls with a shared expert: 10
+// tokens for all is within 0.1% of the best line over its sizes.
 // Below 0.7 items per CU only the four-tile passes are slower (E = 16, I = 512: 25 tokens 32 / 36).
 constexpr double kTiledAlways = 28.0;
 
 inline double tiled_min_tokens(const CallSizes& c) {
   if (static_cast<int64_t>(c.E) * (c.I / 128) * 10 < int64_t{7} * c.cus) return kTiledAlways;
+  if (c.fp8) return 10.0;
   const bool sh = c.Is > 0;
   const int64_t sh_tiles = sh ? (c.T + 255) / 256 : 0;
   const int64_t gate_up = static_cast<int64_t>(c.E) * (c.I / 128) + sh_tiles * (c.Is / 128);
@@ -54,19 +58,10 @@ inline double tiled_min_tokens(const CallSizes& c) {
     const double rounds = static_cast<double>((items + c.cus - 1) / c.cus);
     return std::min(1.2, rounds * c.cus / static_cast<double>(items) - 1.0);
   };
-  const bool part = gate_up < c.cus;
   const double wider = sh ? std::clamp(2.0 * (c.Is - c.I) / c.I, 0.0, 1.0) : 0.0;
-  double t;
-  if (c.fp8) {
-    const bool long_item = sh && gate_up * 10 < int64_t{13} * c.cus &&
-                           (c.T > 256 || c.T % 256 == 0 || c.T % 256 > 128);
-    t = 6.0 + (sh ? 3.0 + 8.0 * idle(gate_up) : 0.0) + (part ? 4.0 : 0.0) + (long_item ? 4.0 : 0.0) +
-        (c.H <= 512 ? 5.0 : 0.0) - 4.0 * wider;
-    return std::clamp(t, 10.0, kTiledAlways);
-  }
-  t = 9.0 + 16.0 * idle(gate_up) + 4.0 * idle(down) + (part ? 8.0 : 0.0) - (c.H <= 512 ? 3.0 : 0.0) -
-      12.0 * wider;
-  return std::clamp(t, 8.0, kTiledAlways);
+  const double t = 8.0 + 16.0 * idle(gate_up) + 4.0 * idle(down) + (gate_up < c.cus ? 6.0 : 0.0) -
+                   8.0 * wider - (c.E >= 128 ? 4.0 : 0.0);
+  return std::clamp(t, gate_up >= 4 * c.cus ? 8.0 : 10.0, kTiledAlways);
 }
 
 // Whether a batch that fits (kInlineRouteTokens, kInlineRouteEntries) is better routed inside the

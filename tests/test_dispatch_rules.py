@@ -1,5 +1,6 @@
 """csrc/rules.hpp, compiled by a host compiler: the line between two kernels of one job takes the side
 that was measured faster (GPU us of the whole call on an MI355X, both sides in one process)."""
+import math
 import os
 import subprocess
 
@@ -19,47 +20,42 @@ def _evaluate(tmp_path, exprs):
     return [float(v) for v in out.split()]
 
 
-# H, E, I, Is, T (8 experts per token), fp8, us streaming, us tiled. Whole rounds of the CUs with and
-# without the shared expert's items past them, partly filled rounds, less than one round, a shared
-# expert wider than the routed ones, short k ranges
+# H, E, I, Is, T (8 experts per token), fp8, us streaming and tiled with uniform routing, the same under a
+# Zipf bias. Whole rounds of the CUs with and without the shared expert's items past them, partly filled
+# rounds, less than one round, a shared expert wider than the routed ones, many and few experts
 MEASURED = [
-    (1024, 64, 512, 256, 137, False, 61.8, 70.4),
-    (512, 128, 384, 0, 241, False, 54.7, 49.8),
-    (512, 128, 256, 256, 209, False, 42.9, 50.1),
-    (512, 48, 512, 512, 103, False, 36.8, 40.9),
-    (512, 160, 256, 512, 341, False, 69.2, 63.9),
-    (512, 100, 512, 0, 188, False, 54.9, 50.3),
-    (512, 96, 512, 256, 181, False, 57.2, 50.1),
-    (512, 128, 384, 512, 241, False, 66.7, 55.5),
-    (512, 100, 768, 256, 188, False, 76.0, 66.3),
-    (512, 160, 768, 0, 481, False, 111.6, 95.2),
-    (1024, 512, 256, 512, 1281, False, 267.4, 193.7),
-    (512, 256, 512, 512, 865, False, 132.3, 112.5),
-    (2048, 100, 384, 0, 163, False, 100.4, 118.8),
-    (2048, 100, 768, 0, 301, False, 211.7, 197.4),
-    (2048, 128, 256, 256, 161, True, 72.9, 82.6),
-    (512, 96, 512, 512, 121, True, 42.4, 45.5),
-    (512, 100, 256, 256, 188, True, 37.0, 40.9),
-    (2048, 64, 512, 256, 81, True, 70.3, 77.9),
-    (2048, 64, 512, 512, 81, True, 70.5, 79.9),
-    (2048, 96, 768, 256, 121, True, 112.8, 123.6),
-    (512, 128, 512, 256, 161, True, 48.6, 53.9),
-    (1024, 100, 256, 512, 126, True, 51.3, 57.5),
-    (512, 48, 512, 512, 73, True, 33.3, 36.7),
-    (512, 100, 768, 256, 276, True, 64.7, 54.4),
-    (2048, 128, 256, 0, 161, True, 74.0, 68.3),
-    (2048, 100, 768, 0, 326, True, 161.7, 128.9),
-    (2048, 100, 512, 256, 226, True, 101.9, 94.6),
-    (512, 256, 768, 0, 833, True, 119.9, 104.2),
+    (512, 64, 512, 512, 105, False, 40.5, 47.9, 47.0, 40.0),
+    (512, 32, 768, 0, 69, False, 34.7, 38.0, 43.6, 42.0),
+    (512, 48, 512, 512, 103, False, 36.8, 40.9, 45.1, 40.0),
+    (2048, 160, 512, 0, 261, False, 191.7, 187.2, 212.8, 105.6),
+    (1024, 160, 256, 0, 341, False, 74.6, 76.7, 115.0, 58.1),
+    (512, 96, 256, 512, 157, False, 49.1, 48.4, 54.3, 45.1),
+    (512, 128, 384, 512, 209, False, 64.2, 55.1, 75.0, 45.8),
+    (2048, 96, 384, 512, 205, False, 121.8, 115.0, 163.8, 85.1),
+    (512, 256, 512, 0, 417, False, 98.5, 92.0, 122.2, 53.8),
+    (512, 512, 512, 512, 641, False, 175.8, 171.2, 182.7, 61.0),
+    (2048, 96, 768, 256, 205, False, 190.1, 186.8, 237.2, 136.2),
+    (2048, 512, 128, 0, 1089, False, 213.7, 192.9, 397.7, 108.2),
+    (512, 96, 512, 512, 205, False, 55.7, 53.7, 70.1, 46.5),
+    (512, 48, 768, 0, 79, False, 42.2, 49.0, 49.4, 43.1),
+    (512, 48, 512, 0, 79, False, 33.0, 35.7, 38.4, 38.5),
+    (512, 96, 256, 256, 157, False, 36.5, 41.0, 45.1, 41.1),
+    (512, 512, 768, 0, 641, True, 158.3, 166.1, 263.4, 64.4),
+    (2048, 96, 768, 0, 121, True, 113.9, 112.8, 158.4, 88.9),
+    (2048, 48, 768, 256, 133, True, 88.7, 80.5, 137.9, 85.6),
+    (1024, 160, 512, 256, 441, True, 99.2, 84.1, 172.6, 63.3),
+    (2048, 128, 512, 256, 161, True, 107.8, 116.0, 162.5, 76.6),
 ]
 
 
-def test_tiled_line_takes_the_measured_side(tmp_path):
+def test_tiled_line_takes_the_faster_side_of_the_mix(tmp_path):
+    """Three uniform calls to one under a bias, by the expected logarithm of the time."""
     got = _evaluate(tmp_path, [
         f"tiled_min_tokens(CallSizes{{{E}, {H}, {I}, {Is}, {T}, {str(fp8).lower()}, 256}})"
-        for H, E, I, Is, T, fp8, _, _ in MEASURED])
-    for (H, E, I, Is, T, fp8, stream, tiled), line in zip(MEASURED, got):
-        assert (T * 8 / E >= line) == (tiled < stream), (H, E, I, Is, T, fp8, line)
+        for H, E, I, Is, T, fp8, *_ in MEASURED])
+    for (H, E, I, Is, T, fp8, us, ut, zs, zt), line in zip(MEASURED, got):
+        gain = 0.75 * math.log(us / ut) + 0.25 * math.log(zs / zt)
+        assert (T * 8 / E >= line) == (gain > 0), (H, E, I, Is, T, fp8, line)
 
 
 # H, E, k, I, Is, T, us with a routing launch, us routed inside gate_up
